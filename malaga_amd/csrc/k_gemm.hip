@@ -97,7 +97,8 @@ hipError_t gemm_simt(const DevMatrix &w, const float *X, int ldx, int M, float *
 
 hipError_t gemm(const DevMatrix &w, const float *X, int ldx, int M, float *Y, int ldy, const float *bias, bool relu,
                 const float *R, int ldr, hipStream_t st, float *ws, size_t ws_bytes) {
-    if (gemm_mfma_supported(w) && ldx % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0)
+    // (the MFMA kernels address a tile's 64 rows of X with 32-bit byte offsets)
+    if (gemm_mfma_supported(w) && ldx % 4 == 0 && ldx < (1 << 24) && reinterpret_cast<uintptr_t>(X) % 16 == 0)
         return gemm_mfma(w, X, ldx, M, Y, ldy, bias, relu, R, ldr, st, ws, ws_bytes);
     return gemm_simt(w, X, ldx, M, Y, ldy, bias, relu, R, ldr, st);
 }

@@ -5,17 +5,18 @@
 // Exactness: the integer quants (q4_K / q5_K nibbles, q6_K 6-bit values - 32,
 // q8_0 int8) are exact in f16, so the MFMA multiplies them by X, which is split
 // into two f16 terms x = hi + lo (|x - hi - lo| <= 2^-22 |x|), with f32
-// accumulation; block scales and k-quant mins are applied per sub-block in f32:
-//   sum_k w_k x_k = d sc * sum_k q_k x_k - dmin m * sum_k x_k,
-// except for q6_K, whose int8 group scales are folded into B as the exact pair
-// bh + bl = q sc (MW<q6_K>::b_split): a super-block's 8 slices of 32 chain in the
-// 16x16x32 MFMA's C operand and d is applied once per block.
+// accumulation.  The block scales go where they cost least VALU work (block_mfma):
+// q4_K / q5_K fold the 6-bit sub-block scale into B (a q, exact in f16), q6_K its int8
+// group scale as the exact pair bh + bl = q sc (MW<q6_K>::b_split), so that a
+// super-block's 8 slices of 32 chain in the 16x16x32 MFMA's C operand and d is applied
+// once per block; the k-quant mins are one more MFMA per block over the 8 sub-block
+// averages of x; q8_0 applies its scale per slice of 32 in f32.
 //
-// Tiling: a workgroup (4 waves) owns 64 rows of W (16 per wave) and BM rows of X.
-// K is consumed in steps of 256 (one k-quant super-block): the X step is staged
-// in LDS as hi/lo f16 plus per-16 sums, while the next step's X and W are in
-// flight in registers.  Each wave keeps its W rows in registers in the MFMA
-// B-operand layout (lane l: row l % 16, k-group l / 16) and reads A (X) from LDS.
+// Tiling: a workgroup of 4 or 8 waves owns BM rows of X and 16 or 32 rows of W per wave
+// (tile_of).  K is consumed in steps of 256 (one k-quant super-block): the X step is staged
+// in LDS as hi/lo f16 (plus the sub-block averages for the formats with mins), while the
+// next step's X and W are in flight in registers.  Each wave keeps its W rows in registers
+// in the MFMA B-operand layout (lane l: row l % 16, k-group l / 16) and reads A (X) from LDS.
 // f16 MFMA operand conversion of quant bytes uses v_perm (byte -> 0x64xx = 1024 +
 // byte) and one packed f16 subtraction.
 #include "kernels.hpp"
@@ -33,11 +34,10 @@ namespace {
 // (k_mfma_rx) uses the same 8-mod-64-dword stride (rx_stride); k_drx keeps K + 8 (its bank
 // conflicts are off the critical path)
 constexpr int kXS = kStep + 16;
+constexpr int kXM = 32;  // halves per row of the sub-block averages (XStage::store)
 
-constexpr int kTileN = 64;        // W rows per workgroup
-
-// X staging of one 256-wide K step into LDS as f16 hi / lo (+ per-16 sums for the
-// formats with mins).  Each thread converts chunks of 8 values and writes them as one
+// X staging of one 256-wide K step into LDS as f16 hi / lo (+ the sub-block averages for
+// the formats with mins).  Each thread converts chunks of 8 values and writes them as one
 // 16-byte store; 16 consecutive lanes take 16 consecutive chunks of one row, so each
 // store of 16 lanes covers 256 contiguous bytes of LDS (no bank conflicts).  Thread t:
 // rows t / 16 + (NTH / 16) u, chunks t % 16 + 16 h (32 chunks per row and step).
@@ -48,35 +48,37 @@ struct XStage {
     static constexpr int R = NTH / 16, RP = BM / R;  // rows per pass, row passes
     static_assert(RP >= 1 && BM % R == 0, "X tile / thread count");
     float4 v[RP][2][2];  // [row pass][chunk h][half]
-    const float *src[RP];
-    bool ok[RP];
+    // a scalar base and a 32-bit lane offset per row (rows past M read row M - 1: their
+    // products are not stored), so that a load needs no vector address arithmetic
+    const char *base;
+    uint32_t off[RP];
     int cl, rg;
     __device__ void init(const float *x, int ldx, int m0, int M, int t) {
         cl = t & 15, rg = t >> 4;
+        base = reinterpret_cast<const char *>(x + size_t(m0) * ldx);
 #pragma unroll
-        for (int u = 0; u < RP; ++u) {
-            const int m = m0 + rg + R * u;
-            ok[u] = m < M;
-            src[u] = x + size_t(ok[u] ? m : 0) * ldx;
-        }
+        for (int u = 0; u < RP; ++u)
+            off[u] = (uint32_t(min(rg + R * u, M - 1 - m0)) * uint32_t(ldx) + uint32_t(koff(cl, 0))) * 4u;
     }
     __device__ static int koff(int c, int half) {
         if constexpr (SPLIT) return 32 * (c >> 2) + 16 * half + 4 * (c & 3);
         else return 8 * c + 4 * half;
     }
     __device__ void load(int kb) {
+        const char *p = base + size_t(kb) * (kStep * 4);
 #pragma unroll
         for (int u = 0; u < RP; ++u)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int f = 0; f < 2; ++f)
-                    v[u][h][f] = ok[u] ? *reinterpret_cast<const float4 *>(src[u] + size_t(kb) * kStep +
-                                                                         koff(cl + 16 * h, f))
-                                       : make_float4(0.f, 0.f, 0.f, 0.f);
+                    v[u][h][f] = *reinterpret_cast<const float4 *>(p + off[u] + 4 * (koff(16 * h, f) - koff(0, 0)));
     }
+    // xm (SUMS): per row the 8 sub-block averages of the step as the A operand of the min
+    // term (block_mfma), kXM halves: [hi of sub-blocks 0..7 | 2048 lo of 0..7 | zeros]
     template <bool SUMS>
-    __device__ void store(_Float16 *xh, _Float16 *xl, float *xsum) const {
+    __device__ void store(_Float16 *xh, _Float16 *xl, _Float16 *xm) const {
+        float sums[RP * 2];
 #pragma unroll
         for (int u = 0; u < RP; ++u)
 #pragma unroll
@@ -85,19 +87,34 @@ struct XStage {
                 const float e[8] = {v[u][h][0].x, v[u][h][0].y, v[u][h][0].z, v[u][h][0].w,
                                     v[u][h][1].x, v[u][h][1].y, v[u][h][1].z, v[u][h][1].w};
                 h8_t hv, lv;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    hv[i] = _Float16(e[i]);
-                    lv[i] = _Float16(e[i] - float(hv[i]));
-                }
+                split_h8(e, hv, lv);
                 *reinterpret_cast<h8_t *>(xh + m * kXS + 8 * c) = hv;
                 *reinterpret_cast<h8_t *>(xl + m * kXS + 8 * c) = lv;
-                if constexpr (SUMS) {  // 16-value sums: this chunk and the next (lane cl ^ 1)
+                if constexpr (SUMS) {  // sums of 32: this chunk and the next three (a quad of lanes)
                     float sm = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
                     sm += dpp_mov<kDppXor1>(sm);
-                    if (!(cl & 1)) xsum[(c >> 1) * BM + m] = sm;
+                    sums[2 * u + h] = sm + dpp_mov<kDppXor2>(sm);
                 }
             }
+        if constexpr (SUMS) {  // lane i of a quad splits and stores the quad's sums i, i + 4, ..
+#pragma unroll
+            for (int k = 0; k < (2 * RP + 3) / 4; ++k) {
+                const int i = 4 * k + (cl & 3);
+                float sm = sums[4 * k];
+#pragma unroll
+                for (int e = 1; e < 4; ++e)
+                    if (4 * k + e < 2 * RP) sm = i == 4 * k + e ? sums[4 * k + e] : sm;
+                sm *= 1.f / 32;  // an average is in the f16 range wherever its values are
+                const _Float16 ah = _Float16(sm), al = _Float16((sm - float(ah)) * 2048.f);
+                _Float16 *p = xm + (rg + R * (i >> 1)) * kXM + (cl >> 2) + 4 * (i & 1);
+                if (2 * RP % 4 == 0 || i < 2 * RP) p[0] = ah, p[8] = al;
+            }
+        }
+    }
+    // the zero half of the xm rows (before the first store; a barrier follows)
+    __device__ static void clear_sums(_Float16 *xm, int t) {
+        for (int i = t; i < BM * 2; i += NTH)
+            *reinterpret_cast<uint4 *>(xm + (i >> 1) * kXM + 16 + 8 * (i & 1)) = make_uint4(0, 0, 0, 0);
     }
 };
 
@@ -110,134 +127,133 @@ struct MfmaArgs {
     const float *bias, *R;
     int ldr, relu;
     float *part;  // split K: raw sums [gridDim.z][M][N], epilogue in k_splitk_reduce
-    int mask_id;  // k_mfma_w MODE 1: row index never selected (-1: none)
-    float *pv;    // k_mfma_w MODE 1: argmax partials [M][parts], one per workgroup
+    int mask_id;  // MODE 1: row index never selected (-1: none)
+    float *pv;    // MODE 1: argmax partials [M][parts], one per workgroup
     uint32_t *pi;
     int parts;
 };
 
 
-// TL (all three GEMM kernels): W from the tile-major copy a.w.t (q6_K / q4_K)
-template <int T, int BM, bool TL>
-__global__ __launch_bounds__(256) void k_mfma(MfmaArgs a) {
+// acc[j][mt] += one 256-wide K block of W tiles cur[j] (16 rows each, B operand) with the
+// staged X rows (A operand).  Bound by VALU work beside the MFMAs, so the scales stay out of
+// the slices:
+//   FOLD (q4_K / q5_K): B = a_s (q - z), z the middle of the quant range, the block's slices
+//     chain in C; what is left of the mins, sum_s (z d a_s - dmin m_s) sum_s x, is two MFMAs
+//     per tile and block, A = the averages of x (hi | 2048 lo), B = (a_s | a_s / 2048) and
+//     (m_s | m_s / 2048): per block acc += d (C + 32 z S) - 32 dmin M.  (Uncentred, C would
+//     carry the mean of q through the chain: 5.0e-7 off 64 bits instead of 3.3e-7.)
+//   SPLIT (q6_K): B = bh + bl, three MFMAs per slice, d once per block.
+//   f16: the slices of all blocks chain in acc.
+// A fragments of slice s + 1 are read from LDS while slice s runs on the MFMA.
+template <int T, int MT, int WT>
+__device__ __forceinline__ void block_mfma(const typename MW<T>::Regs (&cur)[WT], const _Float16 *xh,
+                                           const _Float16 *xl, const _Float16 *xm, int ln, int kq,
+                                           f4_t (&acc)[WT][MT]) {
     using W = MW<T>;
-    constexpr int MT = BM / 16;     // 16-row tiles of X
-    __shared__ _Float16 xh[BM * kXS], xl[BM * kXS];
-    __shared__ float xsum[16 * BM];  // [16-slice][m]
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int kq = lane >> 4, ln = lane & 15;
-    const int n0 = blockIdx.x * kTileN + 16 * w;
-    const int m0 = blockIdx.y * BM;
-    // K steps [kb0, kb1) of this split
-    const int nsteps = a.w.K / kStep, ks = gridDim.z;
-    const int kb0 = int(blockIdx.z) * nsteps / ks, kb1 = (int(blockIdx.z) + 1) * nsteps / ks;
-
-    XStage<BM, 256, W::SPLIT> xs;
-    xs.init(a.x, a.ldx, m0, a.M, t);
-    auto load_x = [&](int kb) { xs.load(kb); };
-    auto stage_x = [&] { xs.template store<W::MIN>(xh, xl, xsum); };
-
-    f4_t acc[MT];
+    constexpr f4_t zero = {0.f, 0.f, 0.f, 0.f};
+    h8_t ahs[2][MT], als[2][MT];
+    auto read_a = [&](int s, h8_t (&ah)[MT], h8_t (&al)[MT]) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt] = f4_t{0.f, 0.f, 0.f, 0.f};
-
-    typename W::Regs cur, nxt;
-    load_w<T, TL>(a.w, n0 >> 4, ln, kb0, kq, cur);
-    load_x(kb0);
-    for (int kb = kb0; kb < kb1; ++kb) {
-        if (kb != kb0) lds_barrier();  // the previous step's reads of xh / xl / xsum are done
-        stage_x();
-        lds_barrier();
-        if (kb + 1 < kb1) {
-            load_w<T, TL>(a.w, n0 >> 4, ln, kb + 1, kq, nxt);
-            load_x(kb + 1);
+        for (int mt = 0; mt < MT; ++mt) {
+            const int xo = (mt * 16 + ln) * kXS + 32 * s + 8 * kq;
+            ah[mt] = *reinterpret_cast<const h8_t *>(xh + xo);
+            al[mt] = *reinterpret_cast<const h8_t *>(xl + xo);
         }
-        if constexpr (W::SPLIT) {
-            // the block's 8 split-B slices chain in the MFMA's C operand; d once per block
-            f4_t cb[MT];
+    };
+    read_a(0, ahs[0], als[0]);
+    [[maybe_unused]] f4_t cb[WT][MT];
+    [[maybe_unused]] FoldPrep fp[WT];
+    if constexpr (W::FOLD) {
 #pragma unroll
-            for (int s = 0; s < W::SLICES32; ++s) {
-                h8_t bh, bl;
-                W::b_split(cur, s, bh, bl);
+        for (int j = 0; j < WT; ++j) fp[j] = fold_prep<W, W::MID_NA>(cur[j]);
+    }
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const int xo = (mt * 16 + ln) * kXS + 32 * s + 8 * kq;
-                    const h8_t ah = *reinterpret_cast<const h8_t *>(xh + xo), al = *reinterpret_cast<const h8_t *>(xl + xo);
-                    cb[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, s ? cb[mt] : f4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    cb[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, cb[mt], 0, 0, 0);
-                    cb[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, cb[mt], 0, 0, 0);
-                }
+    for (int s = 0; s < 8; ++s) {
+        if (s + 1 < 8) read_a(s + 1, ahs[(s + 1) & 1], als[(s + 1) & 1]);
+        if constexpr (W::FOLD || W::SPLIT) {
+            h8_t bh[WT], bl[WT];
+#pragma unroll
+            for (int j = 0; j < WT; ++j) {
+                if constexpr (W::FOLD) bh[j] = W::b_fold_mid(cur[j], fp[j], s);
+                else W::b_split(cur[j], s, bh[j], bl[j]);
             }
-            const float d = W::d_of(cur);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[mt][r] = fmaf(d, cb[mt][r], acc[mt][r]);
+                for (int j = 0; j < WT; ++j)
+                    cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahs[s & 1][mt], bh[j], s ? cb[j][mt] : zero, 0, 0, 0);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int j = 0; j < WT; ++j)
+                    cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(als[s & 1][mt], bh[j], cb[j][mt], 0, 0, 0);
+            if constexpr (W::SPLIT) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int j = 0; j < WT; ++j)
+                        cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahs[s & 1][mt], bl[j], cb[j][mt], 0, 0, 0);
+            }
         } else {
+            float sc[WT], mn[WT];
+            h8_t bop[WT];
 #pragma unroll
-            for (int s = 0; s < W::SLICES; ++s) {
-                float sc, mn;
-                W::scale(cur, s, sc, mn);
-                const auto bop = W::b(cur, s);
+            for (int j = 0; j < WT; ++j) {
+                W::scale(cur[j], s, sc[j], mn[j]);
+                bop[j] = W::b(cur[j], s);
+            }
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const int xo = (mt * 16 + ln) * kXS + s * W::SK + kq * (W::SK / 4);
-                    f4_t tmp = f4_t{0.f, 0.f, 0.f, 0.f};
-                    if constexpr (W::SK == 32) {
-                        const h8_t ah = *reinterpret_cast<const h8_t *>(xh + xo), al = *reinterpret_cast<const h8_t *>(xl + xo);
-                        tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bop, tmp, 0, 0, 0);
-                        tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bop, tmp, 0, 0, 0);
-                    } else {
-                        const h4_t ah = *reinterpret_cast<const h4_t *>(xh + xo), al = *reinterpret_cast<const h4_t *>(xl + xo);
-                        tmp = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, bop, tmp, 0, 0, 0);
-                        tmp = __builtin_amdgcn_mfma_f32_16x16x16f16(al, bop, tmp, 0, 0, 0);
-                    }
-                    // output rows m = mt 16 + 4 kq + r of this lane; x sums of the slice
-                    if constexpr (W::MIN) {
-                        const float *xsp = xsum + (s * W::SK / 16) * BM + mt * 16 + 4 * kq;
-                        float4 xsv = *reinterpret_cast<const float4 *>(xsp);
-                        if constexpr (W::SK == 32) {
-                            const float4 x2 = *reinterpret_cast<const float4 *>(xsp + BM);
-                            xsv = make_float4(xsv.x + x2.x, xsv.y + x2.y, xsv.z + x2.z, xsv.w + x2.w);
-                        }
-                        acc[mt][0] = fmaf(sc, tmp[0], fmaf(-mn, xsv.x, acc[mt][0]));
-                        acc[mt][1] = fmaf(sc, tmp[1], fmaf(-mn, xsv.y, acc[mt][1]));
-                        acc[mt][2] = fmaf(sc, tmp[2], fmaf(-mn, xsv.z, acc[mt][2]));
-                        acc[mt][3] = fmaf(sc, tmp[3], fmaf(-mn, xsv.w, acc[mt][3]));
-                    } else {
+            for (int mt = 0; mt < MT; ++mt) {
+                const h8_t ah = ahs[s & 1][mt], al = als[s & 1][mt];
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[mt][r] = fmaf(sc, tmp[r], acc[mt][r]);
-                    }
+                for (int j = 0; j < WT; ++j) {
+                    f4_t tmp = W::UNIT ? acc[j][mt] : zero;
+                    tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bop[j], tmp, 0, 0, 0);
+                    tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bop[j], tmp, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[j][mt][r] = W::UNIT ? tmp[r] : fmaf(sc[j], tmp[r], acc[j][mt][r]);
                 }
             }
         }
-        cur = nxt;
     }
-    const int n = n0 + ln;
-    if (n >= a.w.N) return;
-    if (a.part) {
-        float *pp = a.part + size_t(blockIdx.z) * a.M * a.w.N;
+    if constexpr (W::FOLD) {
+        // B of the two terms: k-group 0 the 8 scales (mins), k-group 1 those / 2048 (against
+        // the scaled lo parts), k-groups 2 and 3 meet the zeros of A
+        const _Float16 f = kq == 1 ? _Float16(1.f / 2048) : _Float16(1.f);
+        const h8_t f8 = {f, f, f, f, f, f, f, f};
+        h8_t ba[WT], bm[WT];
+        float d[WT], ds[WT], dm[WT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = m0 + mt * 16 + 4 * kq + r;
-                if (m < a.M) pp[size_t(m) * a.w.N + n] = acc[mt][r];
-            }
-        return;
-    }
-    const float bv = a.bias ? a.bias[n] : 0.f;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = m0 + mt * 16 + 4 * kq + r;
-            if (m >= a.M) continue;
-            float v = acc[mt][r] + bv;
-            if (a.R) v += a.R[size_t(m) * a.ldr + n];
-            if (a.relu) v = fmaxf(v, 0.f);
-            a.y[size_t(m) * a.ldy + n] = v;
+        for (int j = 0; j < WT; ++j) {
+            ba[j] = __builtin_bit_cast(h8_t, make_uint4(fp[j].a[0], fp[j].a[1], fp[j].a[2], fp[j].a[3])) * f8;
+            bm[j] = __builtin_bit_cast(h8_t, make_uint4(fp[j].m[0], fp[j].m[1], fp[j].m[2], fp[j].m[3])) * f8;
+            d[j] = h2f(cur[j].hdr.x);
+            ds[j] = float(32 * W::MID) * d[j];
+            dm[j] = -32.f * h2f(cur[j].hdr.x >> 16);
         }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const h8_t am = *reinterpret_cast<const h8_t *>(xm + (mt * 16 + ln) * kXM + 8 * kq);
+#pragma unroll
+            for (int j = 0; j < WT; ++j) {
+                const f4_t sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, ba[j], zero, 0, 0, 0);
+                const f4_t mb = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[j], zero, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    acc[j][mt][r] += fmaf(d[j], cb[j][mt][r], fmaf(ds[j], sb[r], dm[j] * mb[r]));
+            }
+        }
+    } else if constexpr (W::SPLIT) {
+#pragma unroll
+        for (int j = 0; j < WT; ++j) {
+            const float d = W::d_of(cur[j]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[j][mt][r] = fmaf(d, cb[j][mt][r], acc[j][mt][r]);
+        }
+    }
 }
 
 // y[m][n] = sum_{z < ks} part[z][m][n] (in order) + bias[n] (+ R[m][n]) (relu)
@@ -261,43 +277,37 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float *part, int ks
     y[size_t(m) * ldy + n] = v;
 }
 
-// ------------------------------------------------------------- wide tiles
+// ------------------------------------------------------------- tile kernel
 //
-// For large N at M > 32 (the LM head and FFN of batched decode, encoder prefill):
-// 8 waves, each owning WT 16-row tiles of W, so a workgroup covers 128 WT rows of
-// W and one staging of X per K step (f32 -> f16 hi/lo in LDS, x sums) serves
-// 2 WT times more rows than in k_mfma.  A wave reads each X fragment from LDS once
-// per slice and uses it for its WT tiles.
-constexpr int kWWaves = 8;
-
+// NW waves, each owning WT 16-row tiles of W: a workgroup covers 16 NW WT rows of W and BM
+// rows of X, and one staging of X per K step serves all its waves.  A wave reads each X
+// fragment from LDS once per slice and uses it for its WT tiles.
 template <int BM>
-constexpr size_t mfma_w_lds() {
-    return size_t(2) * BM * kXS * sizeof(_Float16) + size_t(16) * BM * sizeof(float);
+constexpr size_t mfma_lds() {
+    return (size_t(2) * BM * kXS + size_t(BM) * kXM) * sizeof(_Float16);
 }
 
 // MODE 0 stores Y (or split-K partials); MODE 1 (the greedy LM head of 33..64 rows) keeps
 // a (value, lowest index) argmax per X row and workgroup instead (gridDim.y = z = 1).
-template <int T, int BM, int WT, bool TL, int MODE = 0>
-__global__ __launch_bounds__(512) void k_mfma_w(MfmaArgs a) {
+// TL: W from the tile-major copy a.w.t (q6_K / q4_K).
+template <int T, int BM, int NW, int WT, bool TL, int MODE = 0>
+__global__ __launch_bounds__(NW * 64, 2) void k_mfma(MfmaArgs a) {
     using W = MW<T>;
     constexpr int MT = BM / 16;
-    constexpr int NTH = kWWaves * 64;
+    constexpr int NTH = NW * 64;
     extern __shared__ __align__(16) unsigned char wlds[];
     _Float16 *xh = reinterpret_cast<_Float16 *>(wlds);
     _Float16 *xl = xh + BM * kXS;
-    float *xsum = reinterpret_cast<float *>(xl + BM * kXS);  // [16-slice][m]
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    _Float16 *xm = xl + BM * kXS;  // [BM][kXM]
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int kq = lane >> 4, ln = lane & 15;
-    const int n0 = blockIdx.x * (kWWaves * 16 * WT) + w * 16 * WT;
+    const int n0 = blockIdx.x * (NW * 16 * WT) + w * 16 * WT;
     const int m0 = blockIdx.y * BM;
     const int nsteps = a.w.K / kStep, ks = gridDim.z;
     const int kb0 = int(blockIdx.z) * nsteps / ks, kb1 = (int(blockIdx.z) + 1) * nsteps / ks;
 
     XStage<BM, NTH, W::SPLIT> xs;
     xs.init(a.x, a.ldx, m0, a.M, t);
-    auto load_x = [&](int kb) { xs.load(kb); };
-    auto stage_x = [&] { xs.template store<W::MIN>(xh, xl, xsum); };
-
     f4_t acc[WT][MT];
 #pragma unroll
     for (int j = 0; j < WT; ++j)
@@ -307,113 +317,19 @@ __global__ __launch_bounds__(512) void k_mfma_w(MfmaArgs a) {
     typename W::Regs cur[WT], nxt[WT];
 #pragma unroll
     for (int j = 0; j < WT; ++j) load_w<T, TL>(a.w, (n0 >> 4) + j, ln, kb0, kq, cur[j]);
-    load_x(kb0);
+    xs.load(kb0);
+    if constexpr (W::MIN) xs.clear_sums(xm, t);
     for (int kb = kb0; kb < kb1; ++kb) {
-        if (kb != kb0) lds_barrier();  // the previous step's reads of xh / xl / xsum are done
-        stage_x();
+        if (kb != kb0) lds_barrier();  // the previous step's reads of xh / xl / xm are done
+        xs.template store<W::MIN>(xh, xl, xm);
         lds_barrier();
-        if (kb + 1 < kb1) {
+        // the next step's operands (past the end: the last step's again, never used, so that
+        // no load sits behind a branch)
+        const int kn = min(kb + 1, kb1 - 1);
 #pragma unroll
-            for (int j = 0; j < WT; ++j) load_w<T, TL>(a.w, (n0 >> 4) + j, ln, kb + 1, kq, nxt[j]);
-            load_x(kb + 1);
-        }
-        if constexpr (W::SPLIT) {
-            // the block's 8 split-B slices chain in the MFMA's C operand; d once per block
-            f4_t cb[WT][MT];
-            // A fragments of slice s + 1 are read from LDS while slice s runs on the MFMA
-            h8_t ahs[2][MT], als[2][MT];
-            auto read_a = [&](int s, h8_t (&ah)[MT], h8_t (&al)[MT]) {
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const int xo = (mt * 16 + ln) * kXS + 32 * s + 8 * kq;
-                    ah[mt] = *reinterpret_cast<const h8_t *>(xh + xo);
-                    al[mt] = *reinterpret_cast<const h8_t *>(xl + xo);
-                }
-            };
-            read_a(0, ahs[0], als[0]);
-#pragma unroll
-            for (int s = 0; s < W::SLICES32; ++s) {
-                if (s + 1 < W::SLICES32) read_a(s + 1, ahs[(s + 1) & 1], als[(s + 1) & 1]);
-                h8_t bh[WT], bl[WT];
-#pragma unroll
-                for (int j = 0; j < WT; ++j) W::b_split(cur[j], s, bh[j], bl[j]);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const h8_t ah = ahs[s & 1][mt], al = als[s & 1][mt];
-#pragma unroll
-                    for (int j = 0; j < WT; ++j)
-                        cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[j], s ? cb[j][mt] : f4_t{0.f, 0.f, 0.f, 0.f},
-                                                                          0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < WT; ++j) cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[j], cb[j][mt], 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < WT; ++j) cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[j], cb[j][mt], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < WT; ++j) {
-                const float d = W::d_of(cur[j]);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[j][mt][r] = fmaf(d, cb[j][mt][r], acc[j][mt][r]);
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < W::SLICES; ++s) {
-                float sc[WT], mn[WT];
-                decltype(W::b(cur[0], 0)) bop[WT];
-#pragma unroll
-                for (int j = 0; j < WT; ++j) {
-                    W::scale(cur[j], s, sc[j], mn[j]);
-                    bop[j] = W::b(cur[j], s);
-                }
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const int xo = (mt * 16 + ln) * kXS + s * W::SK + kq * (W::SK / 4);
-                    float4 xsv = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if constexpr (W::MIN) {
-                        const float *xsp = xsum + (s * W::SK / 16) * BM + mt * 16 + 4 * kq;
-                        xsv = *reinterpret_cast<const float4 *>(xsp);
-                        if constexpr (W::SK == 32) {
-                            const float4 x2 = *reinterpret_cast<const float4 *>(xsp + BM);
-                            xsv = make_float4(xsv.x + x2.x, xsv.y + x2.y, xsv.z + x2.z, xsv.w + x2.w);
-                        }
-                    }
-                    // acc += sc tmp (- mn xsum for the formats with mins)
-                    auto scale_add = [&](f4_t &a4, const f4_t &tmp, float scj, float mnj) {
-                        if constexpr (W::MIN) {
-                            a4[0] = fmaf(scj, tmp[0], fmaf(-mnj, xsv.x, a4[0]));
-                            a4[1] = fmaf(scj, tmp[1], fmaf(-mnj, xsv.y, a4[1]));
-                            a4[2] = fmaf(scj, tmp[2], fmaf(-mnj, xsv.z, a4[2]));
-                            a4[3] = fmaf(scj, tmp[3], fmaf(-mnj, xsv.w, a4[3]));
-                        } else {
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) a4[r] = fmaf(scj, tmp[r], a4[r]);
-                        }
-                    };
-                    if constexpr (W::SK == 32) {
-                        const h8_t ah = *reinterpret_cast<const h8_t *>(xh + xo), al = *reinterpret_cast<const h8_t *>(xl + xo);
-#pragma unroll
-                        for (int j = 0; j < WT; ++j) {
-                            f4_t tmp = f4_t{0.f, 0.f, 0.f, 0.f};
-                            tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bop[j], tmp, 0, 0, 0);
-                            tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bop[j], tmp, 0, 0, 0);
-                            scale_add(acc[j][mt], tmp, sc[j], mn[j]);
-                        }
-                    } else {
-                        const h4_t ah = *reinterpret_cast<const h4_t *>(xh + xo), al = *reinterpret_cast<const h4_t *>(xl + xo);
-#pragma unroll
-                        for (int j = 0; j < WT; ++j) {
-                            f4_t tmp = f4_t{0.f, 0.f, 0.f, 0.f};
-                            tmp = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, bop[j], tmp, 0, 0, 0);
-                            tmp = __builtin_amdgcn_mfma_f32_16x16x16f16(al, bop[j], tmp, 0, 0, 0);
-                            scale_add(acc[j][mt], tmp, sc[j], mn[j]);
-                        }
-                    }
-                }
-            }
-        }
+        for (int j = 0; j < WT; ++j) load_w<T, TL>(a.w, (n0 >> 4) + j, ln, kn, kq, nxt[j]);
+        xs.load(kn);
+        block_mfma<T, MT, WT>(cur, xh, xl, xm, ln, kq, acc);
 #pragma unroll
         for (int j = 0; j < WT; ++j) cur[j] = nxt[j];
     }
@@ -441,7 +357,7 @@ __global__ __launch_bounds__(512) void k_mfma_w(MfmaArgs a) {
         }
         __syncthreads();
         float *mv = reinterpret_cast<float *>(wlds);                     // [waves][BM]
-        uint32_t *mi = reinterpret_cast<uint32_t *>(mv + kWWaves * BM);  // [waves][BM]
+        uint32_t *mi = reinterpret_cast<uint32_t *>(mv + NW * BM);  // [waves][BM]
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -462,7 +378,7 @@ __global__ __launch_bounds__(512) void k_mfma_w(MfmaArgs a) {
             float v = mv[t];
             uint32_t i = mi[t];
 #pragma unroll
-            for (int w2 = 1; w2 < kWWaves; ++w2) argmax_merge(v, i, mv[w2 * BM + t], mi[w2 * BM + t]);
+            for (int w2 = 1; w2 < NW; ++w2) argmax_merge(v, i, mv[w2 * BM + t], mi[w2 * BM + t]);
             a.pv[size_t(m0 + t) * a.parts + blockIdx.x] = v;
             a.pi[size_t(m0 + t) * a.parts + blockIdx.x] = i;
         }
@@ -498,51 +414,49 @@ __global__ __launch_bounds__(512) void k_mfma_w(MfmaArgs a) {
     }
 }
 
-// W tiles per wave of the wide kernel for (N, M), 0: use k_mfma.  Wide tiles pay
-// off once X (M > 32 rows) is re-staged by many tiles and enough workgroups remain:
-// from 96 wide workgroups (config 4's encoder QKV, N = 3072 at 13 row tiles: 105.9 us on
-// k_mfma -> 35 us; at 48 the K = 4096 FFN-down switches too and slows, 37.4 -> 43.6 us).
-int wide_wt(int N, int M) {
-    if (M <= 32) return 0;
-    const int gy = (M + 63) / 64;
-    // WT = 4 (512 rows) would need more than the 256 registers a wave of a
-    // 512-thread workgroup can hold (spills), so 2 (256 rows)
-    return size_t((N + 255) / 256) * gy >= 96 ? 2 : 0;
+struct Tile {
+    int bm, nw, wt;
+    int cols() const { return 16 * nw * wt; }
+    int blocks(int N, int M) const { return (N + cols() - 1) / cols() * ((M + bm - 1) / bm); }
+};
+// The tile for a product: 256 columns of W per workgroup, so that X is staged least often,
+// where the tiles and K splits (split_k) can give every CU a workgroup, else 64 columns.
+// Measured (us, 256 / 64 columns): q4_K 8192 x 2048 at 1651 rows 159 / 192, q6_K 1024 x 4096 at
+// 911 rows 38.8 / 43.6, q4_K 4096 x 1024 at 203 rows 13.7 / 14.2; below the line q4_K
+// 1024 x 1024 at 911 rows 17.1 / 15.9.
+Tile tile_of(const DevMatrix &w, int M) {
+    if (M <= 16) return {16, 4, 1};
+    if (M <= 32) return {32, 4, 1};
+    const Tile wide{64, 8, 2};
+    return int64_t(wide.blocks(w.N, M)) * (w.K / kStep) >= 256 ? wide : Tile{64, 4, 1};
 }
 
-template <int T, int BM, int WT, bool TL, int MODE = 0>
-hipError_t launch_w_t(const MfmaArgs &a, int M, int ks, hipStream_t st) {
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mfma_w<T, BM, WT, TL, MODE>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       int(mfma_w_lds<BM>()));
+template <int T, int BM, int NW, int WT, bool TL, int MODE = 0>
+hipError_t launch_t(const MfmaArgs &a, int ks, hipStream_t st) {
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mfma<T, BM, NW, WT, TL, MODE>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, int(mfma_lds<BM>()));
     if (attr != hipSuccess) return attr;
-    const int gx = (a.w.N + 128 * WT - 1) / (128 * WT);
-    hipLaunchKernelGGL((k_mfma_w<T, BM, WT, TL, MODE>), dim3(gx, (M + BM - 1) / BM, ks), dim3(kWWaves * 64),
-                       mfma_w_lds<BM>(), st, a);
+    hipLaunchKernelGGL((k_mfma<T, BM, NW, WT, TL, MODE>),
+                       dim3((a.w.N + 16 * NW * WT - 1) / (16 * NW * WT), (a.M + BM - 1) / BM, ks), dim3(NW * 64),
+                       mfma_lds<BM>(), st, a);
     return hipGetLastError();
 }
 
 template <int T, bool TL>
-hipError_t launch_tl(const MfmaArgs &a, int M, int ks, hipStream_t st) {
-    if (wide_wt(a.w.N, M) == 2) return launch_w_t<T, 64, 2, TL>(a, M, ks, st);
-    const int gx = (a.w.N + kTileN - 1) / kTileN;
-    if (M <= 16) {
-        hipLaunchKernelGGL((k_mfma<T, 16, TL>), dim3(gx, (M + 15) / 16, ks), dim3(256), 0, st, a);
-    } else if (M <= 32) {
-        hipLaunchKernelGGL((k_mfma<T, 32, TL>), dim3(gx, 1, ks), dim3(256), 0, st, a);
-    } else {
-        hipLaunchKernelGGL((k_mfma<T, 64, TL>), dim3(gx, (M + 63) / 64, ks), dim3(256), 0, st, a);
-    }
-    return hipGetLastError();
+hipError_t launch_tl(const MfmaArgs &a, const Tile &t, int ks, hipStream_t st) {
+    if (t.bm == 16) return launch_t<T, 16, 4, 1, TL>(a, ks, st);
+    if (t.bm == 32) return launch_t<T, 32, 4, 1, TL>(a, ks, st);
+    return t.nw == 4 ? launch_t<T, 64, 4, 1, TL>(a, ks, st) : launch_t<T, 64, 8, 2, TL>(a, ks, st);
 }
 
 // q6_K / q4_K with its tile-major copy reads that copy
 template <int T>
-hipError_t launch(const MfmaArgs &a, int M, int ks, hipStream_t st) {
+hipError_t launch(const MfmaArgs &a, const Tile &t, int ks, hipStream_t st) {
     if constexpr (T == GGML_Q6_K || T == GGML_Q4_K) {
-        if (a.w.t) return launch_tl<T, true>(a, M, ks, st);
+        if (a.w.t) return launch_tl<T, true>(a, t, ks, st);
     }
-    return launch_tl<T, false>(a, M, ks, st);
+    return launch_tl<T, false>(a, t, ks, st);
 }
 
 // Split-K reduction fused with the decoder's residual add and the next LayerNorm
@@ -611,13 +525,15 @@ __global__ __launch_bounds__(256) void k_splitk_qkv(const float *part, int ks, i
     }
 }
 
-// K splits that bring the grid to about one workgroup per CU, within the workspace
+// K splits that fill the device, within the workspace: the 64-row tiles as many as fit in one
+// resident round (one workgroup of 8 waves per CU, two of 4; one split more would start a
+// second round: q6_K 1024 x 4096 at 911 rows 39.6 us with 300 workgroups, 33.4 with 240), the
+// small ones to at least one workgroup per CU
 int split_k(const DevMatrix &w, int M, size_t ws_bytes) {
-    const int wt = wide_wt(w.N, M);
-    const int gx = wt ? (w.N + 128 * wt - 1) / (128 * wt) : (w.N + kTileN - 1) / kTileN;
-    const int bm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
-    const int base = gx * ((M + bm - 1) / bm), nsteps = w.K / kStep;
-    int ks = base >= 256 ? 1 : std::min(nsteps, (256 + base - 1) / base);
+    const Tile t = tile_of(w, M);
+    const int base = t.blocks(w.N, M), nsteps = w.K / kStep;
+    const int fill = t.bm < 64 ? (256 + base - 1) / base : (t.nw == 8 ? 256 : 512) / base;
+    int ks = base >= 256 ? 1 : std::max(1, std::min(nsteps, fill));
     while (ks > 1 && size_t(ks) * M * w.N * sizeof(float) > ws_bytes) --ks;
     return ks;
 }
@@ -720,11 +636,7 @@ __global__ __launch_bounds__(kRxWaves * 64) void k_mfma_rx(RxArgs a) {
                 const float e[8] = {v[u][0].x, v[u][0].y, v[u][0].z, v[u][0].w,
                                     v[u][1].x, v[u][1].y, v[u][1].z, v[u][1].w};
                 h8_t hv, lv;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    hv[i] = _Float16(e[i]);
-                    lv[i] = _Float16(e[i] - float(hv[i]));
-                }
+                split_h8(e, hv, lv);
                 *reinterpret_cast<h8_t *>(xh + m * XS + 8 * cc) = hv;
                 *reinterpret_cast<h8_t *>(xl + m * XS + 8 * cc) = lv;
                 if constexpr (W::MIN) {  // 16-value sums: this chunk and the next (lane t ^ 1)
@@ -1041,14 +953,15 @@ constexpr int kWArgmaxMaxRows = 64;
 bool w_argmax_rows(const DevMatrix &w, int M) {
     return !gemm_rx_supported(w, M) && gemm_mfma_supported(w) && M > 32 && M <= kWArgmaxMaxRows;
 }
-int w_argmax_grid(const DevMatrix &w) { return (w.N + 256 - 1) / 256; }  // WT = 2: 256 rows of W per workgroup
+constexpr Tile kWArgmaxTile{64, 8, 2};  // X is staged least often
+int w_argmax_grid(const DevMatrix &w) { return kWArgmaxTile.blocks(w.N, 1); }
 
 template <int T>
 hipError_t launch_w_argmax(const MfmaArgs &a, int M, hipStream_t st) {
     if constexpr (T == GGML_Q6_K || T == GGML_Q4_K) {
-        if (a.w.t) return launch_w_t<T, 64, 2, true, 1>(a, M, 1, st);
+        if (a.w.t) return launch_t<T, 64, 8, 2, true, 1>(a, 1, st);
     }
-    return launch_w_t<T, 64, 2, false, 1>(a, M, 1, st);
+    return launch_t<T, 64, 8, 2, false, 1>(a, 1, st);
 }
 }  // namespace
 
@@ -1119,11 +1032,11 @@ hipError_t gemm_mfma(const DevMatrix &w, const float *X, int ldx, int M, float *
     a.part = ks > 1 ? ws : nullptr;
     hipError_t e;
     switch (w.type) {
-    case GGML_Q4_K: e = launch<GGML_Q4_K>(a, M, ks, st); break;
-    case GGML_Q5_K: e = launch<GGML_Q5_K>(a, M, ks, st); break;
-    case GGML_Q6_K: e = launch<GGML_Q6_K>(a, M, ks, st); break;
-    case GGML_Q8_0: e = launch<GGML_Q8_0>(a, M, ks, st); break;
-    case GGML_F16: e = launch<GGML_F16>(a, M, ks, st); break;
+    case GGML_Q4_K: e = launch<GGML_Q4_K>(a, tile_of(w, M), ks, st); break;
+    case GGML_Q5_K: e = launch<GGML_Q5_K>(a, tile_of(w, M), ks, st); break;
+    case GGML_Q6_K: e = launch<GGML_Q6_K>(a, tile_of(w, M), ks, st); break;
+    case GGML_Q8_0: e = launch<GGML_Q8_0>(a, tile_of(w, M), ks, st); break;
+    case GGML_F16: e = launch<GGML_F16>(a, tile_of(w, M), ks, st); break;
     default: return hipErrorInvalidValue;
     }
     if (e != hipSuccess || ks == 1) return e;
@@ -1151,11 +1064,11 @@ int launch_split(const DevMatrix &w, const float *X, int ldx, int M, hipStream_t
     a.M = M;
     a.part = ws;
     switch (w.type) {
-    case GGML_Q4_K: *err = launch<GGML_Q4_K>(a, M, ks, st); break;
-    case GGML_Q5_K: *err = launch<GGML_Q5_K>(a, M, ks, st); break;
-    case GGML_Q6_K: *err = launch<GGML_Q6_K>(a, M, ks, st); break;
-    case GGML_Q8_0: *err = launch<GGML_Q8_0>(a, M, ks, st); break;
-    case GGML_F16: *err = launch<GGML_F16>(a, M, ks, st); break;
+    case GGML_Q4_K: *err = launch<GGML_Q4_K>(a, tile_of(w, M), ks, st); break;
+    case GGML_Q5_K: *err = launch<GGML_Q5_K>(a, tile_of(w, M), ks, st); break;
+    case GGML_Q6_K: *err = launch<GGML_Q6_K>(a, tile_of(w, M), ks, st); break;
+    case GGML_Q8_0: *err = launch<GGML_Q8_0>(a, tile_of(w, M), ks, st); break;
+    case GGML_F16: *err = launch<GGML_F16>(a, tile_of(w, M), ks, st); break;
     default: return 1;
     }
     return ks;

@@ -28,6 +28,29 @@ __device__ __forceinline__ uint2 bytes_to_h4(uint32_t v, h2_t off) {
     return make_uint2(bytes_to_h2(v, 0x04010400u, off), bytes_to_h2(v, 0x04030402u, off));
 }
 
+// x - float(half SEL of the f16 pair h): one mixed-precision FMA (the compiler rewrites the
+// multiplication by -1 as a conversion and a subtraction); exact where x - h is
+template <int SEL>
+__device__ __forceinline__ float sub_half(float x, h2_t h) {
+    float r;
+    if constexpr (SEL == 0) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    return r;
+}
+
+// x[0..7] as f16 hi + lo: hi = f16(x), lo = f16(x - hi), both rounded to nearest even
+// (packed conversions: 2 VALU per value instead of 4)
+__device__ __forceinline__ void split_h8(const float (&e)[8], h8_t &hv, h8_t &lv) {
+    typedef float f2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const h2_t h = __builtin_convertvector(f2_t{e[i], e[i + 1]}, h2_t);
+        const h2_t l = __builtin_convertvector(f2_t{sub_half<0>(e[i], h), sub_half<1>(e[i + 1], h)}, h2_t);
+        hv[i] = h[0], hv[i + 1] = h[1];
+        lv[i] = l[0], lv[i + 1] = l[1];
+    }
+}
+
 template <int T>
 struct MW;  // per-type W fetch for one 256-wide K step
 
@@ -43,17 +66,21 @@ struct MW;  // per-type W fetch for one 256-wide K step
 // one packed FMA per pair of values, fma(1024 + q, a, -1024 a) = q a: v_perm gives 1024 + q
 // exactly, (1024 + 15) * 63 <= 65504 stays finite, and the result q a <= 945 is exact.
 // q5_K (q <= 31 would overflow that product) subtracts 1024 first and then multiplies.
+// The prefill GEMMs centre the quants (b_fold_mid): B = a (q - MID).  1032 a is no f16
+// number, so q4_K's pairs there are 64 + q (the nibble in the mantissa's bits 4..7) and
+// na = -72 a, exact as a multiple of 8 below 8192.
 struct FoldPrep {
     uint32_t a[4], na[4], m[4];
 };
 // the k-quant header's 6-bit scales a_j and mins m_j (j < 8, get_scale_min_k4 in ggml's
 // k-quants) for all 8 sub-blocks at once, bytewise: j < 4 from the low 6 bits of bytes j,
 // j + 4; j >= 4 from the nibbles of byte j + 4 and the top 2 bits of bytes j - 4, j
+template <int NA = 1024>
 __device__ __forceinline__ FoldPrep k4_fold_prep(const uint4 &hdr) {
     const uint32_t a03 = hdr.y & 0x3F3F3F3Fu, m03 = hdr.z & 0x3F3F3F3Fu;
     const uint32_t a47 = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
     const uint32_t m47 = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
-    const h2_t off = {_Float16(1024), _Float16(1024)}, neg = {_Float16(-1024), _Float16(-1024)};
+    const h2_t off = {_Float16(1024), _Float16(1024)}, neg = {_Float16(-NA), _Float16(-NA)};
     const uint2 a0 = bytes_to_h4(a03, off), a1 = bytes_to_h4(a47, off);
     const uint2 m0 = bytes_to_h4(m03, off), m1 = bytes_to_h4(m47, off);
     FoldPrep p;
@@ -69,9 +96,9 @@ __device__ __forceinline__ h2_t splat_half(uint32_t u, int h) {
     return h ? __builtin_shufflevector(v, v, 1, 1) : __builtin_shufflevector(v, v, 0, 0);
 }
 
-template <class W>
+template <class W, int NA = 1024>
 __device__ __forceinline__ FoldPrep fold_prep(const typename W::Regs &r) {
-    return k4_fold_prep(r.hdr);
+    return k4_fold_prep<NA>(r.hdr);
 }
 
 template <class W>
@@ -135,6 +162,20 @@ struct MW<GGML_Q4_K> {
     }
     static constexpr bool FOLD = true;
     static constexpr bool SPLIT = false;
+    // B = a_s (q - MID) with na = -MID_NA a_s: v_perm's 64 + q times a_s, minus 72 a_s
+    static constexpr int MID = 8, MID_NA = 72;
+    __device__ static h8_t b_fold_mid(const Regs &r, const FoldPrep &p, int s) {
+        const uint2 q = r.q[s >> 1];
+        const int sh = s & 1 ? 0 : 4;
+        const uint32_t v0 = (q.x << sh) & 0xF0F0F0F0u, v1 = (q.y << sh) & 0xF0F0F0F0u;
+        const h2_t a = splat_half(p.a[s >> 1], s & 1), na = splat_half(p.na[s >> 1], s & 1);
+        auto pair = [&](uint32_t v, uint32_t sel) {
+            const h2_t raw = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x54545454u, v, sel));
+            return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(raw, a, na));
+        };
+        return __builtin_bit_cast(h8_t, make_uint4(pair(v0, 0x04010400u), pair(v0, 0x04030402u), pair(v1, 0x04010400u),
+                                                   pair(v1, 0x04030402u)));
+    }
     // B = a_s q of slice s (FoldPrep): v_perm's 1024 + q times a_s, minus 1024 a_s, in one FMA
     __device__ static h8_t b_fold(const Regs &r, const FoldPrep &p, int s) {
         const uint2 q = r.q[s >> 1];
@@ -167,10 +208,11 @@ struct MW<GGML_Q5_K> {
 #pragma unroll
         for (int g = 0; g < 4; ++g) r.q[g] = *reinterpret_cast<const uint2 *>(blk + 48 + 32 * g + 8 * kq);
     }
+    template <int OFF = 1024>
     __device__ static h8_t b(const Regs &r, int s) {
         const uint2 q = r.q[s >> 1];
         const int sh = 4 * (s & 1);
-        const h2_t off = {_Float16(1024), _Float16(1024)};
+        const h2_t off = {_Float16(OFF), _Float16(OFF)};
         const uint32_t v0 = ((q.x >> sh) & 0x0F0F0F0Fu) | (((r.qh.x >> s) & 0x01010101u) << 4);
         const uint32_t v1 = ((q.y >> sh) & 0x0F0F0F0Fu) | (((r.qh.y >> s) & 0x01010101u) << 4);
         const uint2 lo = bytes_to_h4(v0, off), hi = bytes_to_h4(v1, off);
@@ -187,6 +229,12 @@ struct MW<GGML_Q5_K> {
         const h2_t a = splat_half(p.a[s >> 1], s & 1);
         const h8_t av = __builtin_shufflevector(a, a, 0, 1, 0, 1, 0, 1, 0, 1);
         return b(r, s) * av;
+    }
+    static constexpr int MID = 16, MID_NA = 1024;
+    __device__ static h8_t b_fold_mid(const Regs &r, const FoldPrep &p, int s) {
+        const h2_t a = splat_half(p.a[s >> 1], s & 1);
+        const h8_t av = __builtin_shufflevector(a, a, 0, 1, 0, 1, 0, 1, 0, 1);
+        return b<1024 + MID>(r, s) * av;
     }
 };
 
@@ -281,6 +329,7 @@ struct MW<GGML_Q8_0> {
     static constexpr bool MIN = false;
     static constexpr bool FOLD = false;
     static constexpr bool SPLIT = false;
+    static constexpr bool UNIT = false;
     struct Regs {
         uint2 q[8];
         uint4 d;  // 8 f16 scales
@@ -310,6 +359,7 @@ struct MW<GGML_F16> {
     static constexpr bool MIN = false;
     static constexpr bool FOLD = false;
     static constexpr bool SPLIT = false;
+    static constexpr bool UNIT = true;  // the scale is 1: slices chain in the MFMA's C operand
     struct Regs {
         uint4 q[8];
     };

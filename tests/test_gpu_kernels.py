@@ -147,6 +147,30 @@ def test_gemm_wide_tiles(ctx, t, N, K):
         ctx.lib.mlg_matrix_free(w)
 
 
+@pytest.mark.parametrize("t", (Q4_K, Q5_K, Q6_K, Q8_0, F16))
+@pytest.mark.parametrize("M_,N,K", [(33, 16, 256), (65, 255, 512), (129, 257, 1024), (64, 8192, 256), (127, 4100, 512)])
+def test_gemm_tile_edges(ctx, t, M_, N, K):
+    """One row or column past and short of the 64-row / 256- and 64-column tiles, on both sides
+    of the tile rule and with K split or not; the k-quant mins and the centred quants (a MFMA
+    over the sub-block averages of x) also with same-sign activations near the top of the f16
+    range, whose sums of 32 are beyond it."""
+    rng = np.random.default_rng(M_ + N + t)
+    blocks = M.quantize(t, rng.normal(0, 0.02, (N, K)).astype(np.float32))
+    w = upload(ctx, t, blocks, N, K)
+    try:
+        wd = O.dequant(t, blocks, N * K).reshape(N, K)
+        for lo, hi in ((-1, 1), (1e-3, 2e-3), (3e4, 6e4)):
+            x = rng.uniform(lo, hi, (M_, K)).astype(np.float32)
+            xd, yd = dev(x), torch.zeros((M_, N), device="cuda")
+            _lib.check(ctx.lib.mlg_gemm(w, ptr(xd), M_, ptr(yd), None, 0, None))
+            torch.cuda.synchronize()
+            # 2e-6 of sum |x| |w| as above; x below the normal range of the f16 lo part keeps 3e-8
+            lim = 2e-6 * bound(x, wd) + 3e-8 * np.abs(wd).sum(1)
+            assert (np.abs(yd.cpu().numpy() - O.gemv(t, blocks, N, K, x)) <= lim).all(), (lo, hi)
+    finally:
+        ctx.lib.mlg_matrix_free(w)
+
+
 @pytest.mark.parametrize("t,K", [(Q6_K, 1024), (Q4_K, 1024), (Q8_0, 512), (Q5_K, 2048), (Q6_K, 2048)])
 def test_gemm_argmax_batched_lm_head(ctx, t, K):
     """Batched LM head (5..64 rows): per-workgroup argmax partials merged on the host equal
