@@ -303,6 +303,42 @@ hipError_t step_cross_attn(const DevMatrix &wq, const float *bq, const DevMatrix
 // y = x W^T + bias, x [nb][K] in global memory.
 hipError_t step_proj(const DevMatrix &w, const float *bias, int nb, const float *x, float *y, hipStream_t st);
 
+// ---- all decoder layers of a batch-1 step in one resident launch, k_resident.hip ----
+struct ResMat {
+    const uint8_t *q, *s, *d;  // DevMatrix planes
+    const float *bias;
+};
+struct ResNorm {
+    const float *g, *b;
+};
+struct ResLayer {
+    ResMat qkv, out, cq, cout, up, down;
+    ResNorm attn_norm, cross_norm, ffn_norm;
+};
+struct ResStep {
+    const ResLayer *layers;  // device array [L]
+    int L, d, f, H, m, s;
+    uint32_t proj;           // type of the projections (FFN down and the embedding: q6_K)
+    uint64_t *words;         // step_resident_words(..) of this state, zero before the first launch
+    uint32_t *epoch;         // 1 before the first launch; each launch leaves it one higher
+    uint32_t *flag;          // 0; set when a launch could not finish its waits (its results are void)
+    uint32_t spins;          // polls per wait
+    const DevMatrix *emb;    // input row: emb[ids[0]], or the source token src says
+    const uint32_t *ids;
+    SrcEmb src;
+    const float *pos;
+    uint32_t pos_base;
+    float emb_scale, eps;
+    const uint32_t *step, *lens;
+    __half *kv, *ckv;        // self / cross caches of every layer: K then V, [H][m or s][hd]
+    float *x_out, *y;        // x before the last FFN output, and that output (bias added)
+};
+// The shapes and types it covers; the device must hold its grid at once (step_resident_fits).
+bool step_resident_supported(int d, int f, int H, int hd, int layers, uint32_t proj, uint32_t down, uint32_t emb);
+bool step_resident_fits(int d, int H, uint32_t proj, int device);
+size_t step_resident_words(int d, int f, int layers);
+hipError_t step_resident(const ResStep &r, hipStream_t st);
+
 // *p += 1 on the device.
 hipError_t inc_u32(uint32_t *p, hipStream_t st);
 // Fill n uint32 values (graph-safe replacement for hipMemsetAsync).

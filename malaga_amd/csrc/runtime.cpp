@@ -524,7 +524,42 @@ void Model::load(const std::string &path) {
         check_hip(hipMemcpy(sl->d_ids, sl->ids.data(), size_t(n) * 4, hipMemcpyHostToDevice), "upload");
         shortlists.push_back(std::move(sl));
     }
+    build_resident();
     check_hip(hipDeviceSynchronize(), "model upload");
+}
+
+// The layer table of the resident batch-1 step, where its kernel covers the model (one type
+// for all projections) and the device.  MALAGA_RESIDENT_STEP=0 keeps the per-layer launches;
+// MALAGA_RESIDENT_SPINS sets the polls per wait (a test hook; 2^20 are about a second).
+void Model::build_resident() {
+    const char *off = std::getenv("MALAGA_RESIDENT_STEP");
+    if (dec.empty() || no_fuse_ || split_cross_ || (off && std::string(off) == "0")) return;
+    const uint32_t proj = dec[0].qkv.w.type;
+    const int L = int(dec.size()), H = cfg.decoder_heads;
+    if (!step_resident_supported(cfg.d_model, cfg.decoder_ffn, H, cfg.d_model / H, L, proj, dec[0].down.w.type,
+                                 embed.type) ||
+        !step_resident_fits(cfg.d_model, H, proj, ctx->device))
+        return;
+    auto mat = [](const Linear &l) { return ResMat{l.w.q, l.w.s, l.w.d, l.b}; };
+    auto norm = [](const LNorm &n) { return ResNorm{n.g, n.b}; };
+    std::vector<ResLayer> table;
+    for (const DecLayer &l : dec) {
+        for (const Linear *p : {&l.qkv, &l.out, &l.cross_q, &l.cross_out, &l.up})
+            if (p->w.type != proj) return;
+        if (l.down.w.type != dec[0].down.w.type) return;
+        table.push_back({mat(l.qkv), mat(l.out), mat(l.cross_q), mat(l.cross_out), mat(l.up), mat(l.down),
+                         norm(l.attn_norm), norm(l.cross_norm), norm(l.ffn_norm)});
+    }
+    ResLayer *t = static_cast<ResLayer *>(dev_alloc(table.size() * sizeof(ResLayer), "layer table"));
+    owned_.push_back(t);
+    check_hip(hipMemcpy(t, table.data(), table.size() * sizeof(ResLayer), hipMemcpyHostToDevice), "upload");
+    const char *spins = std::getenv("MALAGA_RESIDENT_SPINS");
+    res_spins_ = spins ? uint32_t(std::strtoul(spins, nullptr, 10)) : 1u << 20;
+    res_layers_ = t;
+}
+
+bool Model::resident_ok(const DevMatrix &emb, int b, int m, int s) const {
+    return res_layers_ && b == 1 && emb.type == GGML_Q6_K && fusable(b, m, s);
 }
 
 void Model::ensure_embed() {
@@ -713,7 +748,7 @@ std::unique_ptr<Batch> Model::encode(const std::vector<std::vector<uint32_t>> &s
 }
 
 std::unique_ptr<StaticState> Model::new_state(int b, int s, int m, bool logits, bool row_map, const Shortlist *sl,
-                                              bool kv32) {
+                                              bool kv32, bool resident) {
     auto st = std::make_unique<StaticState>();
     st->b = b;
     st->s = s;
@@ -766,6 +801,16 @@ std::unique_ptr<StaticState> Model::new_state(int b, int s, int m, bool logits, 
     if (st->fused) {
         st->part = static_cast<float *>(get(size_t(H) * b * d * 4, "attention partial sums"));
         st->part2 = static_cast<float *>(get(size_t(H) * b * d * 4, "cross attention partial sums"));
+    }
+    st->resident = resident && st->fused;
+    if (st->resident) {
+        const size_t words = step_resident_words(d, cfg.decoder_ffn, L);
+        st->words = static_cast<uint64_t *>(get(words * sizeof(uint64_t), "resident step words"));
+        st->epoch = static_cast<uint32_t *>(get(4, "resident step epoch"));
+        st->res_flag = static_cast<uint32_t *>(get(4, "resident step flag"));
+        check_hip(fill_u32(reinterpret_cast<uint32_t *>(st->words), 0, 2 * words, ctx->stream), "fill");
+        check_hip(fill_u32(st->epoch, 1, 1, ctx->stream), "fill");
+        check_hip(fill_u32(st->res_flag, 0, 1, ctx->stream), "fill");
     }
     if (!st->fused && dgemm_step_ok(b))
         st->lnstat = static_cast<double *>(get(size_t(d / 16) * b * 2 * sizeof(double), "LayerNorm statistics"));
@@ -902,6 +947,23 @@ float *Model::step_fused(StaticState &st, bool final_ln) {
     hipStream_t s = ctx->stream;
     const int B = st.b, d = cfg.d_model, H = cfg.decoder_heads, hd = d / H;
     float *cur = st.x, *nxt = st.xb;
+    if (st.resident) {
+        ResStep r{};
+        r.layers = res_layers_;
+        r.L = int(dec.size()), r.d = d, r.f = cfg.decoder_ffn, r.H = H, r.m = st.m, r.s = st.s;
+        r.proj = dec[0].qkv.w.type;
+        r.words = st.words, r.epoch = st.epoch, r.flag = st.res_flag, r.spins = res_spins_;
+        r.emb = st.sl ? &st.sl->head : &embed;
+        r.ids = st.sl ? st.sl_row : st.ids;
+        if (st.sl) r.src = SrcEmb{st.src_emb, st.src_row, st.s};
+        r.pos = pos, r.pos_base = uint32_t(cfg.pad_token_id + 1), r.emb_scale = embed_scale, r.eps = kLnEps;
+        r.step = st.step, r.lens = st.lens;
+        r.kv = st.kc[0], r.ckv = st.ck[0];
+        r.x_out = cur, r.y = st.y;
+        check_hip(step_resident(r, s), "step_resident");
+        if (final_ln) check_hip(residual_ln(cur, st.y, B, d, dec_norm.g, dec_norm.b, kLnEps, st.h, s), "residual_ln");
+        return cur;
+    }
     for (size_t i = 0; i < dec.size(); ++i) {
         const DecLayer &l = dec[i];
         if (i == 0) {
@@ -1222,6 +1284,26 @@ std::vector<std::vector<uint32_t>> GraphCache::greedy(const Batch &src, uint32_t
     }
 }
 
+namespace {
+// One resident launch at a time on a device: two that each held part of the CUs would wait
+// for CUs the other holds until their polls run out.  A call that finds the turn taken (a
+// thread with another context) decodes with the per-layer launches.
+struct ResidentTurn {
+    static std::atomic<bool> &taken(int device) {
+        static std::atomic<bool> t[64];
+        return t[device & 63];
+    }
+    int device = -1;
+    bool take(int dev) {
+        if (!taken(dev).exchange(true, std::memory_order_acquire)) device = dev;
+        return device >= 0;
+    }
+    ~ResidentTurn() {
+        if (device >= 0) taken(device).store(false, std::memory_order_release);
+    }
+};
+}  // namespace
+
 std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tgt_lang, int max_new, int sync_every,
                                                    bool eos_mask, bool use_graph, const Shortlist *sl,
                                                    std::vector<std::vector<float>> *top) {
@@ -1234,16 +1316,19 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     const int b = capture ? int(next_pow2(uint32_t(n))) : n;
     const int kb = b, ks = bucket(src.s, 16, max_m), km = bucket(max_new + 2, 32, max_m);
     ++clock_;
+    ResidentTurn turn;  // until the stream is drained below
+    const bool resident = m.resident_ok(sl ? sl->head : m.embed, kb, km, ks) && turn.take(m.ctx->device);
     Entry *e = nullptr;
     for (auto &it : entries_)
-        if (it.b == kb && it.s == ks && it.m == km && it.sl == sl) e = &it;
+        if (it.b == kb && it.s == ks && it.m == km && it.sl == sl && it.resident == resident) e = &it;
     if (!e) {
         Entry ne;
         ne.b = kb;
         ne.s = ks;
         ne.m = km;
         ne.sl = sl;
-        ne.st = m.new_state(kb, ks, km, false, false, sl);
+        ne.resident = resident;
+        ne.st = m.new_state(kb, ks, km, false, false, sl, false, resident);
         entries_.push_back(std::move(ne));
         e = &entries_.back();
         evict(e);
@@ -1326,7 +1411,14 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     check_hip(hipMemcpyAsync(out.data(), st.out, out.size() * 4, hipMemcpyDeviceToHost, s), "D2H");
     if (top) check_hip(hipMemcpyAsync(outv.data(), st.outv, outv.size() * 4, hipMemcpyDeviceToHost, s), "D2H");
     check_hip(hipMemcpyAsync(&err, st.err, 4, hipMemcpyDeviceToHost, s), "D2H");
+    uint32_t stuck = 0;
+    if (st.resident) check_hip(hipMemcpyAsync(&stuck, st.res_flag, 4, hipMemcpyDeviceToHost, s), "D2H");
     check_hip(hipStreamSynchronize(s), "sync");
+    if (stuck) {  // the results are void; from here on this model launches per layer
+        m.drop_resident();
+        clear();
+        return run(src, tgt_lang, max_new, sync_every, eos_mask, use_graph, sl, top);
+    }
     if (err) fail(ERR_INVALID, kNonFiniteLogits);
     std::vector<std::vector<uint32_t>> res(static_cast<size_t>(n));
     if (top) top->assign(static_cast<size_t>(n), {});

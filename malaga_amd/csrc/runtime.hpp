@@ -137,6 +137,11 @@ struct StaticState {
     uint8_t *src_q = nullptr;             // lazy embeddings: token_embd rows of src_ids (device layout)
     uint32_t *src_iota = nullptr;         // lazy embeddings: 0 .. b*s-1
     bool fused = false;                   // decoder step uses the fused kernels of k_step.hip
+    // batch-1 greedy: the layers run as one resident launch (k_resident.hip) over these words
+    // (with fused, whose kernels remain the way when that launch could not finish its waits)
+    bool resident = false;
+    uint64_t *words = nullptr;
+    uint32_t *epoch = nullptr, *res_flag = nullptr;
     float *logits = nullptr, *pv = nullptr;
     uint32_t *pi = nullptr;
     int parts = 0;
@@ -178,6 +183,7 @@ class GraphCache {
     struct Entry {
         int b, s, m;
         const Shortlist *sl = nullptr;  // part of the key (src/graph.rs:157)
+        bool resident = false;          // part of the key
         std::unique_ptr<StaticState> st;
         hipGraphExec_t exec = nullptr;
         uint64_t last_used = 0;
@@ -233,7 +239,13 @@ class Model {
     // sl: buffers of shortlist decoding (greedy only).
     // kv32: f32 K/V caches (the generic path; never the fused step kernels)
     std::unique_ptr<StaticState> new_state(int b, int s, int m, bool logits, bool row_map = false,
-                                           const Shortlist *sl = nullptr, bool kv32 = false);
+                                           const Shortlist *sl = nullptr, bool kv32 = false,
+                                           bool resident = false);
+    // Whether a batch-1 greedy state over head `emb` takes the resident launch; its caller
+    // holds the device's one turn for it (GraphCache::run) and decodes again without it when
+    // st.res_flag was raised (drop_resident).
+    bool resident_ok(const DevMatrix &emb, int b, int m, int s) const;
+    void drop_resident() { res_layers_ = nullptr; }
     // src/model.rs:552-612: one decoder step on fixed buffers.  greedy: argmax +
     // bookkeeping, else logits into st.logits and ++step.
     void step(StaticState &st, bool greedy, int mask_id);
@@ -285,6 +297,9 @@ class Model {
     bool dgemm_step_ok(int b) const;
     void step_dgemm(StaticState &st, bool greedy_mode, int mask_id);
     bool split_k_step_ = false;  // MALAGA_SPLIT_K_STEP=1: batches > 4 keep the split-K GEMMs
+    ResLayer *res_layers_ = nullptr;  // device table of the decoder layers (null: no resident step)
+    uint32_t res_spins_ = 0;
+    void build_resident();
     bool no_fuse_ = false;  // MALAGA_NO_FUSED_STEP=1 forces the unfused step
     bool split_cross_ = false;  // MALAGA_SPLIT_CROSS_STEP=1: cross_q and cross attention as two launches
 };

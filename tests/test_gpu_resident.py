@@ -1,0 +1,98 @@
+"""The resident batch-1 decoder step (k_resident.hip): all layers in one launch."""
+import threading
+
+import numpy as np
+import pytest
+
+import malaga_amd as M
+import oracle as O
+from tests.test_gpu_full_size import argmax_chain_check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    d0 = tmp_path_factory.mktemp("resident")
+    made = {}
+
+    def get(preset, d, f, layers=3):
+        p = d0 / f"{preset}-{d}-{f}.gguf"
+        if p not in made:
+            cfg = dict(vocab_size=1200, d_model=d, encoder_layers=1, decoder_layers=layers, encoder_heads=d // 64,
+                       decoder_heads=d // 64, encoder_ffn=512, decoder_ffn=f, max_position_embeddings=256,
+                       max_length=200, scale_embedding=1, bos_token_id=0, pad_token_id=1, eos_token_id=2,
+                       decoder_start_token_id=2)
+            M.write_synthetic(p, cfg, preset, M.INIT_NORMAL_RICH, seed=d + f, std=0.04, name="resident")
+            made[p] = p
+        return p
+
+    return get
+
+
+@pytest.mark.parametrize("preset", ["q4_k_m", "q5_k_m"])
+@pytest.mark.parametrize("d,f", [(256, 512), (512, 1536), (1024, 4096), (1024, 2560)])
+def test_resident_step_matches_oracle(model, preset, d, f):
+    """Every width the kernel takes, FFNs that fill and do not fill the gathering threads, and
+    one key, a few and more keys than one round of the 8 waves (64) in both attentions: each
+    token is the oracle's argmax after the same prefix, the winning logits within 2e-3."""
+    path = model(preset, d, f)
+    gpu, orc = M.Translator.load(path), O.Model(path)
+    try:
+        for n, new in ((1, 5), (7, 9), (70, 72)):
+            src = [np.random.default_rng(n + d).integers(4, 1200, n).tolist()]
+            batch = gpu.encode_cross(src)
+            toks, top = gpu.greedy_top(batch, 1100, new, eos_mask=True)
+            again = gpu.greedy_top(batch, 1100, new, eos_mask=True)  # the captured graph
+            eager = gpu.greedy_top(batch, 1100, new, eos_mask=True, graph=False)
+            assert again == (toks, top) == eager
+            tgt = np.array([[2, 1100] + toks[0][:-1]], np.uint32)
+            ref = orc.teacher_forced_logits(src, tgt, kv_f16=True)
+            argmax_chain_check(toks, top, ref, tie=4e-3)
+    finally:
+        gpu.close()
+
+
+def test_resident_step_off_and_out_of_polls(model, monkeypatch):
+    """MALAGA_RESIDENT_STEP=0 and a launch whose waits run out at once (the flag is raised and
+    the call decodes again per layer, then and from there on) give what the per-layer step
+    gives."""
+    path = model("q4_k_m", 512, 1536)
+    src = [np.random.default_rng(3).integers(4, 1200, 11).tolist()]
+    out = {}
+    for name, env in (("on", {}), ("off", {"MALAGA_RESIDENT_STEP": "0"}), ("stuck", {"MALAGA_RESIDENT_SPINS": "0"})):
+        with monkeypatch.context() as m:
+            for k, v in env.items():
+                m.setenv(k, v)
+            gpu = M.Translator.load(path)
+        batch = gpu.encode_cross(src)
+        out[name] = [gpu.greedy_top(batch, 1100, 20, eos_mask=True) for _ in range(3)]
+        gpu.close()
+    assert out["stuck"] == out["off"]
+    for (a, ta), (b, tb) in zip(out["on"], out["off"]):
+        assert a == b and np.abs(np.array(ta) - np.array(tb)).max() < 1e-3
+
+
+def test_resident_step_from_several_threads(model):
+    """Contexts of their own on one device: one call at a time has the resident launch, the
+    others decode per layer meanwhile; every call gives its own sentence's tokens."""
+    path = model("q4_k_m", 256, 512)
+    srcs = [[np.random.default_rng(50 + i).integers(4, 1200, 4 + 5 * i).tolist()] for i in range(3)]
+    ref = M.Translator.load(path)
+    want = [ref.generate(s, 1100, M.GenOptions(max_new_tokens=30, eos_mask=True)) for s in srcs]
+    ref.close()
+    ts = [M.Translator.load(path) for _ in srcs]
+    done = []
+
+    def work(i):
+        done.append((i, all(ts[i].generate(srcs[i], 1100, M.GenOptions(max_new_tokens=30, eos_mask=True)) == want[i]
+                            for _ in range(8))))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(ts))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(100)
+    assert sorted(done) == [(i, True) for i in range(len(ts))]
+    for t in ts:
+        t.close()
