@@ -649,94 +649,113 @@ __device__ __forceinline__ void top8_insert(Top8 &t, float v, uint32_t i) {
 
 // Pass 1: per (part, row): chunk max M, sum exp(x - M), chunk top-8.
 // work layout per (row, part): [M, S, v0..v7, i0..i7] (18 floats)
+//
+// All 2048 workgroups of 32 x 256206 are resident at once, so a launch lasts as long as one
+// workgroup's chain: with two reads of the chunk, 8 argmax rounds of one wave for the
+// threshold and 8 more over 256 lists it took 25 of the 32.5 us of a call.  Now (R > 0: the
+// chunk fits in R values per thread) the values are read once, the threshold is the least of
+// 8 group maxima, the few values that reach it go to one list, and each takes its place by
+// counting the better ones.
+constexpr int kTopList = 512;  // candidates kept in LDS; more (ties): one sorted list per thread
+
+template <int R>
 __global__ __launch_bounds__(256) void k_lsm_topk_partial(const float *logits, int V, int k, int mask_id,
                                                           float *work) {
-    __shared__ float red[16];
+    __shared__ float red[16], gmax[kTopMax];
     __shared__ float lv[256 * kTopMax];
     __shared__ uint32_t li[256 * kTopMax];
-    const int row = blockIdx.y, p = blockIdx.x, P = gridDim.x;
+    __shared__ uint32_t count;
+    static_assert(kTopList <= 256 * kTopMax, "the candidates share the lists' space");
+    const int row = blockIdx.y, p = blockIdx.x, P = gridDim.x, t = threadIdx.x;
     const int chunk = (V + P - 1) / P, start = p * chunk, end = min(start + chunk, V);
     const float *r = logits + size_t(row) * V;
-    __shared__ float thv;
-    __shared__ uint32_t thx;
-    // pass 1: the thread's own best (value, index) and the chunk's max
-    float bv = -INFINITY;
-    uint32_t bx = 0xffffffffu;
-    for (int i = start + threadIdx.x; i < end; i += blockDim.x) {
-        if (i == mask_id) continue;
-        const float v = r[i];
-        if (better(v, uint32_t(i), bv, bx)) {
-            bv = v;
-            bx = uint32_t(i);
-        }
-    }
-    lv[threadIdx.x] = bv;
-    li[threadIdx.x] = bx;
-    const float mx = block_max(bv, red);  // its barrier also orders lv / li
-    // the chunk's 8 best are all at least as good as the 8th best of the 256 threads' bests
-    // (8 distinct elements): wave 0 finds that threshold ((-inf, ~0) below 8 elements)
-    if (threadIdx.x < 64) {  // wave-uniform
-        const int lane = threadIdx.x;
-        float hv[4];
-        uint32_t hx[4];
+    // element j of this thread is start + t + 256 j; f(value, index) of every unmasked one
+    float x[R > 0 ? R : 1];
+    if constexpr (R > 0)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            hv[q] = lv[64 * q + lane];
-            hx[q] = li[64 * q + lane];
-        }
-        float wv = -INFINITY;
-        uint32_t wx = 0xffffffffu;
+        for (int j = 0; j < R; ++j) x[j] = r[min(start + t + 256 * j, V - 1)];
+    auto each = [&](auto &&f) {
+        if constexpr (R > 0) {
 #pragma unroll
-        for (int rr = 0; rr < kTopMax; ++rr) {
-            wv = hv[0];
-            wx = hx[0];
-#pragma unroll
-            for (int q = 1; q < 4; ++q)
-                if (better(hv[q], hx[q], wv, wx)) {
-                    wv = hv[q];
-                    wx = hx[q];
-                }
-            wave_argmax(wv, wx);
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (hx[q] == wx) {
-                    hv[q] = -INFINITY;
-                    hx[q] = 0xffffffffu;
-                }
+            for (int j = 0; j < R; ++j) {
+                const int i = start + t + 256 * j;
+                if (i < end && i != mask_id) f(x[j], uint32_t(i));
+            }
+        } else {
+            for (int i = start + t; i < end; i += 256)
+                if (i != mask_id) f(r[i], uint32_t(i));
         }
-        if (lane == 0) {
-            thv = wv;
-            thx = wx;
-        }
-    }
+    };
+    float best = -INFINITY;
+    each([&](float v, uint32_t) { best = v > best ? v : best; });
+    // the maxima of 8 groups of 32 threads are 8 distinct values of the chunk, so its 8 best
+    // are all at least the least of them (-inf where a group has no value)
+    const float half = group_reduce(best, 5, OpMax{});
+    if ((t & 31) == 0) gmax[t >> 5] = half;
+    if (t == 0) count = 0u;
     __syncthreads();
-    const float tv = thv;
-    const uint32_t tx = thx;
-    // pass 2: sum exp(x - max), and a sorted top-8 of the thread's elements that reach the
-    // threshold (a handful per workgroup)
-    Top8 t;
-    top8_init(t);
-    float s = 0.f;
-    for (int i = start + threadIdx.x; i < end; i += blockDim.x) {
-        if (i == mask_id) continue;
-        const float v = r[i];
-        if (mx > -INFINITY) s += expf(v - mx);
-        if (!better(tv, tx, v, uint32_t(i))) top8_insert(t, v, uint32_t(i));
+    float thr = gmax[0], mx = gmax[0];
+#pragma unroll
+    for (int g = 1; g < kTopMax; ++g) {
+        thr = fminf(thr, gmax[g]);
+        mx = fmaxf(mx, gmax[g]);
     }
-    s = block_sum(s, red);
-    // the workgroup's best 8: the 256 sorted lists in LDS, entry e of list L at e 256 + L
+    // sum exp(x - max), and the values that reach the threshold (two dozen of 4004)
+    float s = 0.f;
+    each([&](float v, uint32_t i) {
+        if (mx > -INFINITY) s += expf(v - mx);
+        if (v >= thr) {
+            const uint32_t at = atomicAdd(&count, 1u);
+            if (at < uint32_t(kTopList)) {
+                lv[at] = v;
+                li[at] = i;
+            }
+        }
+    });
+    s = block_sum(s, red);  // its barriers order the list
+    float *o = work + (size_t(row) * P + p) * (2 + 2 * kTopMax);
+    if (t == 0) {
+        o[0] = mx;
+        o[1] = s;
+    }
+    const int n = int(count);
+    if (n <= kTopList) {
+        // the order is total (value, then lower index): a candidate's place is the number of
+        // better ones, whatever order the list was filled in
+        for (int c = t; c < n; c += 256) {
+            const float v = lv[c];
+            const uint32_t i = li[c];
+            int rank = 0;
+            for (int q = 0; q < n; ++q) rank += better(lv[q], li[q], v, i) ? 1 : 0;
+            if (rank < kTopMax) {
+                o[2 + rank] = v;
+                o[2 + kTopMax + rank] = __uint_as_float(i);
+            }
+        }
+        if (t >= n && t < kTopMax) {
+            o[2 + t] = -INFINITY;
+            o[2 + kTopMax + t] = __uint_as_float(0xffffffffu);
+        }
+        return;
+    }
+    // many ties: each thread's sorted 8 best in LDS, entry e of list L at e 256 + L
     // (consecutive lanes, consecutive banks), then wave 0 takes the best head of all lists
     // 8 times: lane l keeps the heads of lists l + 64 q in registers and reads a list's next
-    // entry only when its head wins.  The order is total (value, then lower index), so the
-    // result is the 8 best whatever the merge order.
+    // entry only when its head wins
+    __syncthreads();
+    Top8 top;
+    top8_init(top);
+    each([&](float v, uint32_t i) {
+        if (v >= thr) top8_insert(top, v, i);
+    });
 #pragma unroll
     for (int j = 0; j < kTopMax; ++j) {
-        lv[j * 256 + threadIdx.x] = t.v[j];
-        li[j * 256 + threadIdx.x] = t.i[j];
+        lv[j * 256 + t] = top.v[j];
+        li[j * 256 + t] = top.i[j];
     }
     __syncthreads();
-    if (threadIdx.x >= 64) return;  // wave-uniform; no barrier below
-    const int lane = threadIdx.x;
+    if (t >= 64) return;  // wave-uniform; no barrier below
+    const int lane = t;
     int head[4];
     float hv[4];
     uint32_t hx[4];
@@ -746,10 +765,8 @@ __global__ __launch_bounds__(256) void k_lsm_topk_partial(const float *logits, i
         hv[q] = lv[64 * q + lane];
         hx[q] = li[64 * q + lane];
     }
-    float ov[kTopMax];
-    uint32_t oi[kTopMax];
 #pragma unroll
-    for (int r = 0; r < kTopMax; ++r) {
+    for (int e8 = 0; e8 < kTopMax; ++e8) {
         float bv = hv[0];
         uint32_t bx = hx[0];
 #pragma unroll
@@ -759,8 +776,10 @@ __global__ __launch_bounds__(256) void k_lsm_topk_partial(const float *logits, i
                 bx = hx[q];
             }
         wave_argmax(bv, bx);
-        ov[r] = bv;
-        oi[r] = bx;
+        if (lane == 0) {
+            o[2 + e8] = bv;
+            o[2 + kTopMax + e8] = __uint_as_float(bx);
+        }
         // the list whose head won moves on (indices are unique; padding entries are -inf)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -769,16 +788,6 @@ __global__ __launch_bounds__(256) void k_lsm_topk_partial(const float *logits, i
                 hv[q] = e < kTopMax ? lv[e * 256 + 64 * q + lane] : -INFINITY;
                 hx[q] = e < kTopMax ? li[e * 256 + 64 * q + lane] : 0xffffffffu;
             }
-    }
-    if (lane == 0) {
-        float *o = work + (size_t(row) * P + p) * (2 + 2 * kTopMax);
-        o[0] = mx;
-        o[1] = s;
-#pragma unroll
-        for (int j = 0; j < kTopMax; ++j) {
-            o[2 + j] = ov[j];
-            o[2 + kTopMax + j] = __uint_as_float(oi[j]);
-        }
     }
 }
 
@@ -1153,7 +1162,12 @@ size_t logsoftmax_topk_scratch(int rows, int k) {
 hipError_t logsoftmax_topk(const float *logits, int rows, int V, int k, int mask_id, float *work, float *vals,
                            uint32_t *idx, hipStream_t st) {
     if (k < 1 || k > kTopMax) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_lsm_topk_partial, dim3(kTopParts, rows), dim3(256), 0, st, logits, V, k, mask_id, work);
+    // 16 values per thread cover chunks of 4096 (vocabularies up to 262144); beyond, the chunk
+    // is read again for each use
+    if ((V + kTopParts - 1) / kTopParts <= 16 * 256)
+        hipLaunchKernelGGL(k_lsm_topk_partial<16>, dim3(kTopParts, rows), dim3(256), 0, st, logits, V, k, mask_id, work);
+    else
+        hipLaunchKernelGGL(k_lsm_topk_partial<0>, dim3(kTopParts, rows), dim3(256), 0, st, logits, V, k, mask_id, work);
     hipLaunchKernelGGL(k_lsm_topk_final, dim3(rows), dim3(64), 0, st, work, rows, kTopParts, k, vals, idx);
     return hipGetLastError();
 }

@@ -453,6 +453,31 @@ def test_logsoftmax_topk(ctx):
     assert idx.cpu().numpy()[3].tolist() == [10, 11, 12, 13]
 
 
+@pytest.mark.parametrize("V", [5, 63, 64, 700, 16384, 16385, 262144, 262145])
+def test_logsoftmax_topk_lists(ctx, V):
+    """Chunks that leave threads, groups and parts without a value, chunks on both sides of 16
+    values per thread, more ties than the candidate list holds (every value equal; two values
+    only), and rows of -inf but a few: the 8 best by value, then lower index."""
+    rng = np.random.default_rng(V)
+    k = min(8, V)
+    x = rng.normal(0, 2, (5, V)).astype(np.float32)
+    x[1] = 1.5
+    x[2] = rng.integers(0, 2, V)
+    x[3, rng.permutation(V)[k:]] = -np.inf
+    x[4] = np.sort(x[4])
+    xd = dev(x)
+    scratch = torch.zeros(ctx.lib.mlg_logsoftmax_topk_scratch(5, k) // 4 + 1, device="cuda")
+    vals, idx = torch.zeros((5, k), device="cuda"), torch.zeros((5, k), dtype=torch.int32, device="cuda")
+    _lib.check(ctx.lib.mlg_logsoftmax_topk(ptr(xd), 5, V, k, -1, ptr(scratch), ptr(vals), ptr(idx), None))
+    torch.cuda.synchronize()
+    xx = x.astype(np.float64)
+    order = np.lexsort((np.tile(np.arange(V), (5, 1)), -xx), axis=1)[:, :k]
+    lse = np.log(np.exp(xx - xx.max(1, keepdims=True)).sum(1)) + xx.max(1)
+    np.testing.assert_array_equal(idx.cpu().numpy(), order)
+    # 2^-24 of |x - max| and ln of up to 2.6e5 terms, f32
+    np.testing.assert_allclose(vals.cpu().numpy(), np.take_along_axis(xx, order, 1) - lse[:, None], atol=2e-5)
+
+
 def test_attention_rejects_unsupported_head_size(ctx):
     q = torch.zeros(1, 48, device="cuda")
     kv = torch.zeros(1, 1, 4, 48, dtype=torch.float16, device="cuda")
