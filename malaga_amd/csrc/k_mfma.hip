@@ -580,7 +580,7 @@ size_t rx_lds_bytes(int BM, int K) {
     return size_t(BM) * rx_stride(K) * 2 * sizeof(_Float16) + size_t(K / 16) * BM * sizeof(float);
 }
 
-template <int T, int BM, int MODE, bool TL>
+template <int T, int BM, int MODE, bool TL, bool NT>
 __global__ __launch_bounds__(kRxWaves * 64) void k_mfma_rx(RxArgs a) {
     using W = MW<T>;
     constexpr int MT = BM / 16;
@@ -602,7 +602,7 @@ __global__ __launch_bounds__(kRxWaves * 64) void k_mfma_rx(RxArgs a) {
     auto job_base = [&](int j) { return (gw + (j / nsteps) * nw) * 16 * kRxNT; };
     auto load_job = [&](int j, typename W::Regs (&r)[kRxNT]) {
 #pragma unroll
-        for (int nt = 0; nt < kRxNT; ++nt) load_w<T, TL>(a.w, (job_base(j) >> 4) + nt, ln, j % nsteps, kq, r[nt]);
+        for (int nt = 0; nt < kRxNT; ++nt) load_w<T, TL, NT>(a.w, (job_base(j) >> 4) + nt, ln, j % nsteps, kq, r[nt]);
     };
 
     // stage X: chunks of 8 values, one 16-byte store each (consecutive lanes: consecutive
@@ -864,24 +864,32 @@ __global__ __launch_bounds__(kRxWaves * 64) void k_mfma_rx(RxArgs a) {
 }
 
 // Dynamic LDS beyond 64 KB needs the kernel attribute raised once.
-template <int T, int BM, int MODE, bool TL>
+template <int T, int BM, int MODE, bool TL, bool NT>
 hipError_t launch_rx_bm(const RxArgs &a, int grid, hipStream_t st) {
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mfma_rx<T, BM, MODE, TL>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mfma_rx<T, BM, MODE, TL, NT>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(kRxMaxLds));
     if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL((k_mfma_rx<T, BM, MODE, TL>), dim3(grid), dim3(kRxWaves * 64), rx_lds_bytes(BM, a.w.K), st,
+    hipLaunchKernelGGL((k_mfma_rx<T, BM, MODE, TL, NT>), dim3(grid), dim3(kRxWaves * 64), rx_lds_bytes(BM, a.w.K), st,
                        a);
     return hipGetLastError();
 }
 
-template <int T, int MODE, bool TL>
+template <int T, int MODE, bool TL, bool NT = false>
 hipError_t launch_rx_tl(const RxArgs &a, int M, int grid, hipStream_t st) {
-    return M <= 16 ? launch_rx_bm<T, 16, MODE, TL>(a, grid, st) : launch_rx_bm<T, 32, MODE, TL>(a, grid, st);
+    return M <= 16 ? launch_rx_bm<T, 16, MODE, TL, NT>(a, grid, st) : launch_rx_bm<T, 32, MODE, TL, NT>(a, grid, st);
 }
 
 template <int T, int MODE>
 hipError_t launch_rx(const RxArgs &a, int M, int grid, hipStream_t st) {
     if constexpr (T == GGML_Q6_K || T == GGML_Q4_K) {
+        // The greedy head of the 600M vocabulary (221 MB of tiles) cannot stay in the 256 MB
+        // Infinity Cache beside the layers' 112 MB, and read with ordinary loads it evicts them
+        // once per step: non-temporal, 32 sentences of 32 tokens took 21.66 instead of 22.35
+        // ms.  (Logits are stored by ordinary loads: alone, over and over, they are faster with
+        // what the cache keeps, 67 against 72 us.)
+        if constexpr (T == GGML_Q6_K && MODE == 1)
+            if (a.w.t && size_t(a.w.N) * a.w.nb * (kQ6TileBytes / 16) > size_t(32) << 20)
+                return launch_rx_tl<T, MODE, true, true>(a, M, grid, st);
         if (a.w.t) return launch_rx_tl<T, MODE, true>(a, M, grid, st);
     }
     return launch_rx_tl<T, MODE, false>(a, M, grid, st);

@@ -269,17 +269,20 @@ struct MW<GGML_Q6_K> {
     }
     // the same registers from the tile-major copy (kQ6TileBytes per tile and block):
     // five loads, each of whole cache lines, instead of fourteen of 16 scattered rows
+    // (NT: non-temporal, a head too large to stay in the Infinity Cache)
+    template <bool NT = false>
     __device__ static void load_tile(const uint8_t *tw, int nb, int tile, int kb, int kq, int ln, Regs &r) {
         const uint8_t *tb = tw + (size_t(tile) * nb + kb) * kQ6TileBytes;
         const int li = 16 * kq + ln;
-        const uint4 a = *reinterpret_cast<const uint4 *>(tb + 16 * li);
-        const uint4 b = *reinterpret_cast<const uint4 *>(tb + 1024 + 16 * li);
-        const uint4 h = *reinterpret_cast<const uint4 *>(tb + 2048 + 16 * li);
+        const uint4 a = ld_u4<NT>(tb + 16 * li);
+        const uint4 b = ld_u4<NT>(tb + 1024 + 16 * li);
+        const uint4 h = ld_u4<NT>(tb + 2048 + 16 * li);
         r.qa[0] = a.x, r.qa[1] = a.y, r.qa[2] = a.z, r.qa[3] = a.w;
         r.qb[0] = b.x, r.qb[1] = b.y, r.qb[2] = b.z, r.qb[3] = b.w;
         r.qh[0] = h.x, r.qh[1] = h.y, r.qh[2] = h.z, r.qh[3] = h.w;
-        r.sc = *reinterpret_cast<const uint4 *>(tb + 3072 + 16 * ln);
-        r.d = *reinterpret_cast<const unsigned short *>(tb + 3328 + 2 * ln);
+        r.sc = ld_u4<NT>(tb + 3072 + 16 * ln);
+        if constexpr (NT) r.d = __builtin_nontemporal_load(reinterpret_cast<const unsigned short *>(tb + 3328 + 2 * ln));
+        else r.d = *reinterpret_cast<const unsigned short *>(tb + 3328 + 2 * ln);
     }
     __device__ static h4_t b(const Regs &r, int G) {
         const int n = G >> 3, t = (G >> 1) & 3, h = G & 1, nh = 2 * n + h;
@@ -377,9 +380,10 @@ struct MW<GGML_F16> {
 
 // W registers of row 16 tile + ln, K block kb: from the tile-major copy (TL, q6_K / q4_K; a
 // tile past the last reads the last) or from the planes (the row clamped to N - 1)
-template <int T, bool TL>
+template <int T, bool TL, bool NT = false>
 __device__ __forceinline__ void load_w(const WPtr &w, int tile, int ln, int kb, int kq, typename MW<T>::Regs &r) {
-    if constexpr (TL) MW<T>::load_tile(w.t, w.nb, min(tile, (w.N + 15) / 16 - 1), kb, kq, ln, r);
+    if constexpr (NT) MW<T>::template load_tile<true>(w.t, w.nb, min(tile, (w.N + 15) / 16 - 1), kb, kq, ln, r);
+    else if constexpr (TL) MW<T>::load_tile(w.t, w.nb, min(tile, (w.N + 15) / 16 - 1), kb, kq, ln, r);
     else MW<T>::load(w, min(16 * tile + ln, w.N - 1), kb, kq, r);
 }
 
