@@ -138,12 +138,14 @@ struct MfmaArgs {
 // staged X rows (A operand).  Bound by VALU work beside the MFMAs, so the scales stay out of
 // the slices:
 //   FOLD (q4_K / q5_K): B = a_s (q - z), z the middle of the quant range, the block's slices
-//     chain in C; what is left of the mins, sum_s (z d a_s - dmin m_s) sum_s x, is two MFMAs
-//     per tile and block, A = the averages of x (hi | 2048 lo), B = (a_s | a_s / 2048) and
-//     (m_s | m_s / 2048): per block acc += d (C + 32 z S) - 32 dmin M.  (Uncentred, C would
-//     carry the mean of q through the chain: 5.0e-7 off 64 bits instead of 3.3e-7.)
+//     chain in C; what is left of the mins, sum_s T_s sum_s x with T_s = z d a_s - dmin m_s, is
+//     one MFMA per tile and block over the averages of x (hi | 2048 lo | hi): per block
+//     acc += d C + 32 T.  Neither C nor T carries the mean of the weights, which cancels
+//     (off 64 bits, x of zero mean / after ReLU: scales and mins per slice in f32 3.0e-7 /
+//     5.4e-7, uncentred 5.0e-7, centred with separate sums of a_s x and m_s x 2.0e-7 / 9.1e-7).
 //   SPLIT (q6_K): B = bh + bl, three MFMAs per slice, d once per block.
-//   f16: the slices of all blocks chain in acc.
+//   q8_0, f16: the slice's scale (1) in f32 (chained in acc, f16 would round twice per slice:
+//     1.6e-7 off 64 bits instead of 1.1e-7).
 // A fragments of slice s + 1 are read from LDS while slice s runs on the MFMA.
 template <int T, int MT, int WT>
 __device__ __forceinline__ void block_mfma(const typename MW<T>::Regs (&cur)[WT], const _Float16 *xh,
@@ -207,41 +209,52 @@ __device__ __forceinline__ void block_mfma(const typename MW<T>::Regs (&cur)[WT]
                 const h8_t ah = ahs[s & 1][mt], al = als[s & 1][mt];
 #pragma unroll
                 for (int j = 0; j < WT; ++j) {
-                    f4_t tmp = W::UNIT ? acc[j][mt] : zero;
+                    f4_t tmp = zero;
                     tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bop[j], tmp, 0, 0, 0);
                     tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bop[j], tmp, 0, 0, 0);
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        acc[j][mt][r] = W::UNIT ? tmp[r] : fmaf(sc[j], tmp[r], acc[j][mt][r]);
+                        acc[j][mt][r] = fmaf(sc[j], tmp[r], acc[j][mt][r]);
                 }
             }
         }
     }
     if constexpr (W::FOLD) {
-        // B of the two terms: k-group 0 the 8 scales (mins), k-group 1 those / 2048 (against
-        // the scaled lo parts), k-groups 2 and 3 meet the zeros of A
-        const _Float16 f = kq == 1 ? _Float16(1.f / 2048) : _Float16(1.f);
-        const h8_t f8 = {f, f, f, f, f, f, f, f};
-        h8_t ba[WT], bm[WT];
-        float d[WT], ds[WT], dm[WT];
+        // T_s = z d a_s - dmin m_s, what is left of the mins, as an f16 pair: exact products and
+        // one rounding in f32, scaled by 64 / p (p: the power of two below the larger of z d and
+        // dmin) so that |T| <= 16128 and T / 2048 stays normal.  k-groups of the MFMA: Thi with
+        // the averages' hi, Thi / 2048 with 2048 lo, Tlo with hi again, zeros.
+        h8_t bt[WT];
+        float d[WT], back[WT];
 #pragma unroll
         for (int j = 0; j < WT; ++j) {
-            ba[j] = __builtin_bit_cast(h8_t, make_uint4(fp[j].a[0], fp[j].a[1], fp[j].a[2], fp[j].a[3])) * f8;
-            bm[j] = __builtin_bit_cast(h8_t, make_uint4(fp[j].m[0], fp[j].m[1], fp[j].m[2], fp[j].m[3])) * f8;
             d[j] = h2f(cur[j].hdr.x);
-            ds[j] = float(32 * W::MID) * d[j];
-            dm[j] = -32.f * h2f(cur[j].hdr.x >> 16);
+            const float dmin = h2f(cur[j].hdr.x >> 16), zd = float(W::MID) * d[j];
+            const uint32_t pb = __float_as_uint(fmaxf(fmaxf(fabsf(zd), fabsf(dmin)), 1e-30f)) & 0x7f800000u;
+            const float inv = __uint_as_float(0x7f000000u - pb) * 64.f, da = zd * inv, dm = dmin * inv;
+            back[j] = 0.5f * __uint_as_float(pb);  // 32 p / 64
+            float t[8];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const h2_t av = __builtin_bit_cast(h2_t, fp[j].a[s >> 1]), mv = __builtin_bit_cast(h2_t, fp[j].m[s >> 1]);
+                t[s] = fmaf(da, float(av[s & 1]), -(dm * float(mv[s & 1])));
+            }
+            h8_t hi, lo;
+            split_h8(t, hi, lo);
+            const _Float16 f = kq == 1 ? _Float16(1.f / 2048) : _Float16(1.f);
+            const h8_t f8 = {f, f, f, f, f, f, f, f};
+            bt[j] = kq < 2 ? hi * f8 : lo;
         }
+        const int ao = kq == 1 ? 8 : kq == 3 ? 16 : 0;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const h8_t am = *reinterpret_cast<const h8_t *>(xm + (mt * 16 + ln) * kXM + 8 * kq);
+            const h8_t am = *reinterpret_cast<const h8_t *>(xm + (mt * 16 + ln) * kXM + ao);
 #pragma unroll
             for (int j = 0; j < WT; ++j) {
-                const f4_t sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, ba[j], zero, 0, 0, 0);
-                const f4_t mb = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[j], zero, 0, 0, 0);
+                const f4_t tb = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bt[j], zero, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    acc[j][mt][r] += fmaf(d[j], cb[j][mt][r], fmaf(ds[j], sb[r], dm[j] * mb[r]));
+                    acc[j][mt][r] = fmaf(back[j], tb[r], fmaf(d[j], cb[j][mt][r], acc[j][mt][r]));
             }
         }
     } else if constexpr (W::SPLIT) {
@@ -420,15 +433,18 @@ struct Tile {
     int blocks(int N, int M) const { return (N + cols() - 1) / cols() * ((M + bm - 1) / bm); }
 };
 // The tile for a product: 256 columns of W per workgroup, so that X is staged least often,
-// where the tiles and K splits (split_k) can give every CU a workgroup, else 64 columns.
-// Measured (us, 256 / 64 columns): q4_K 8192 x 2048 at 1651 rows 159 / 192, q6_K 1024 x 4096 at
-// 911 rows 38.8 / 43.6, q4_K 4096 x 1024 at 203 rows 13.7 / 14.2; below the line q4_K
-// 1024 x 1024 at 911 rows 17.1 / 15.9.
+// where at least 96 such tiles, or those times the K steps that can be split off (split_k),
+// keep the device busy, else 64 columns.  Measured (us, 256 / 64 columns): q4_K 8192 x 2048 at
+// 1651 rows 159 / 192, q6_K 1024 x 4096 at 911 rows 38.8 / 43.6; below the line q4_K 1024 x 1024
+// at 911 rows 17.1 / 15.9.  K is split only where 64-column tiles alone leave CUs idle: the
+// context's workspace is shared by its streams, and products that fill the device without it
+// (q4_K 4096 x 1024 at 203 rows: 13.7 split / 14.2) stay independent of each other.
 Tile tile_of(const DevMatrix &w, int M) {
     if (M <= 16) return {16, 4, 1};
     if (M <= 32) return {32, 4, 1};
-    const Tile wide{64, 8, 2};
-    return int64_t(wide.blocks(w.N, M)) * (w.K / kStep) >= 256 ? wide : Tile{64, 4, 1};
+    const Tile wide{64, 8, 2}, narrow{64, 4, 1};
+    const int nw = wide.blocks(w.N, M);
+    return nw >= 96 || (narrow.blocks(w.N, M) < 256 && int64_t(nw) * (w.K / kStep) >= 256) ? wide : narrow;
 }
 
 template <int T, int BM, int NW, int WT, bool TL, int MODE = 0>

@@ -332,7 +332,6 @@ struct MW<GGML_Q8_0> {
     static constexpr bool MIN = false;
     static constexpr bool FOLD = false;
     static constexpr bool SPLIT = false;
-    static constexpr bool UNIT = false;
     struct Regs {
         uint2 q[8];
         uint4 d;  // 8 f16 scales
@@ -362,7 +361,6 @@ struct MW<GGML_F16> {
     static constexpr bool MIN = false;
     static constexpr bool FOLD = false;
     static constexpr bool SPLIT = false;
-    static constexpr bool UNIT = true;  // the scale is 1: slices chain in the MFMA's C operand
     struct Regs {
         uint4 q[8];
     };
