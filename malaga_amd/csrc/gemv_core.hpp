@@ -182,6 +182,114 @@ __device__ __forceinline__ void load_chunk(const WPtr &w, int row, int c, Raw<T>
     }
 }
 
+// dot4u8 as one asm block: each byte is converted where it is used, so a schedule
+// cannot convert every item's bytes ahead of their products (which overflows the
+// registers of a multi-item dot); same operations, same order
+__device__ __forceinline__ float dot4u8_chain(uint32_t v, const float (&x)[4], float acc) {
+    float t0, t1, t2, t3;
+    asm("v_cvt_f32_ubyte0 %1, %5\n\t"
+        "v_cvt_f32_ubyte1 %2, %5\n\t"
+        "v_fmac_f32 %0, %1, %6\n\t"
+        "v_cvt_f32_ubyte2 %3, %5\n\t"
+        "v_fmac_f32 %0, %2, %7\n\t"
+        "v_cvt_f32_ubyte3 %4, %5\n\t"
+        "v_fmac_f32 %0, %3, %8\n\t"
+        "v_fmac_f32 %0, %4, %9"
+        : "+v"(acc), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+        : "v"(v), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+    return acc;
+}
+
+// dot4u8_chain of four items' words against the same four x values, as one asm block:
+// byte b of every word is converted, then the four products are added, so the four
+// items' dependent chains interleave (one chain per block left each product waiting for
+// the previous one); per item the operations and their order are dot4u8_chain's
+__device__ __forceinline__ void dot4u8_chain4(const uint32_t (&v)[4], const float (&x)[4], float (&acc)[4]) {
+    float t0, t1, t2, t3;
+    asm("v_cvt_f32_ubyte0 %4, %8\n\t"
+        "v_cvt_f32_ubyte0 %5, %9\n\t"
+        "v_cvt_f32_ubyte0 %6, %10\n\t"
+        "v_cvt_f32_ubyte0 %7, %11\n\t"
+        "v_fmac_f32 %0, %4, %12\n\t"
+        "v_fmac_f32 %1, %5, %12\n\t"
+        "v_fmac_f32 %2, %6, %12\n\t"
+        "v_fmac_f32 %3, %7, %12\n\t"
+        "v_cvt_f32_ubyte1 %4, %8\n\t"
+        "v_cvt_f32_ubyte1 %5, %9\n\t"
+        "v_cvt_f32_ubyte1 %6, %10\n\t"
+        "v_cvt_f32_ubyte1 %7, %11\n\t"
+        "v_fmac_f32 %0, %4, %13\n\t"
+        "v_fmac_f32 %1, %5, %13\n\t"
+        "v_fmac_f32 %2, %6, %13\n\t"
+        "v_fmac_f32 %3, %7, %13\n\t"
+        "v_cvt_f32_ubyte2 %4, %8\n\t"
+        "v_cvt_f32_ubyte2 %5, %9\n\t"
+        "v_cvt_f32_ubyte2 %6, %10\n\t"
+        "v_cvt_f32_ubyte2 %7, %11\n\t"
+        "v_fmac_f32 %0, %4, %14\n\t"
+        "v_fmac_f32 %1, %5, %14\n\t"
+        "v_fmac_f32 %2, %6, %14\n\t"
+        "v_fmac_f32 %3, %7, %14\n\t"
+        "v_cvt_f32_ubyte3 %4, %8\n\t"
+        "v_cvt_f32_ubyte3 %5, %9\n\t"
+        "v_cvt_f32_ubyte3 %6, %10\n\t"
+        "v_cvt_f32_ubyte3 %7, %11\n\t"
+        "v_fmac_f32 %0, %4, %15\n\t"
+        "v_fmac_f32 %1, %5, %15\n\t"
+        "v_fmac_f32 %2, %6, %15\n\t"
+        "v_fmac_f32 %3, %7, %15"
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+}
+
+// the same of two items
+__device__ __forceinline__ void dot4u8_chain2(const uint32_t (&v)[2], const float (&x)[4], float (&acc)[2]) {
+    float t0, t1;
+    asm("v_cvt_f32_ubyte0 %2, %4\n\t"
+        "v_cvt_f32_ubyte0 %3, %5\n\t"
+        "v_fmac_f32 %0, %2, %6\n\t"
+        "v_fmac_f32 %1, %3, %6\n\t"
+        "v_cvt_f32_ubyte1 %2, %4\n\t"
+        "v_cvt_f32_ubyte1 %3, %5\n\t"
+        "v_fmac_f32 %0, %2, %7\n\t"
+        "v_fmac_f32 %1, %3, %7\n\t"
+        "v_cvt_f32_ubyte2 %2, %4\n\t"
+        "v_cvt_f32_ubyte2 %3, %5\n\t"
+        "v_fmac_f32 %0, %2, %8\n\t"
+        "v_fmac_f32 %1, %3, %8\n\t"
+        "v_cvt_f32_ubyte3 %2, %4\n\t"
+        "v_cvt_f32_ubyte3 %3, %5\n\t"
+        "v_fmac_f32 %0, %2, %9\n\t"
+        "v_fmac_f32 %1, %3, %9"
+        : "+v"(acc[0]), "+v"(acc[1]), "=&v"(t0), "=&v"(t1)
+        : "v"(v[0]), "v"(v[1]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+}
+template <int KI>
+__device__ __forceinline__ void dot4u8_items(const uint32_t (&v)[KI], const float (&x)[4], float (&acc)[KI]) {
+    if constexpr (KI == 4) {
+        dot4u8_chain4(v, x, acc);
+    } else if constexpr (KI == 2) {
+        dot4u8_chain2(v, x, acc);
+    } else {
+#pragma unroll
+        for (int k = 0; k < KI; ++k) acc[k] = dot4u8_chain(v[k], x, acc[k]);
+    }
+}
+
+// acc + the value of a 64-value q4_K / q5_K chunk: sums al, ah of the products of its two
+// sub-blocks' quants, s0, s1 of their x; and of a q6_K chunk (four groups of 16)
+__device__ __forceinline__ float k4_chunk(float acc, float d, float dmin, float sc0, float m0, float sc1, float m1,
+                                          float al, float ah, float s0, float s1) {
+    acc += d * (sc0 * al + sc1 * ah) - dmin * (m0 * s0 + m1 * s1);
+    return acc;
+}
+__device__ __forceinline__ float q6_chunk(float acc, float d, const float (&sc)[4], const float (&a)[4],
+                                          const float (&s)[4]) {
+    acc += d * (sc[0] * (a[0] - 32.f * s[0]) + sc[1] * (a[1] - 32.f * s[1]) + sc[2] * (a[2] - 32.f * s[2]) +
+                sc[3] * (a[3] - 32.f * s[3]));
+    return acc;
+}
+
 template <int T, int B>
 __device__ __forceinline__ void dot_chunk(int c, const Raw<T> &r, const XF<T, B> &X, float (&acc)[B]) {
     if constexpr (T == GGML_Q4_K || T == GGML_Q5_K) {
@@ -227,7 +335,7 @@ __device__ __forceinline__ void dot_chunk(int c, const Raw<T> &r, const XF<T, B>
                 ah = dot4u8(hi[u], &X.x[bi][32 + 4 * u], ah);
             }
             if constexpr (T == GGML_Q4_K) ah *= 0.0625f;
-            acc[bi] += d * (sc0 * al + sc1 * ah) - dmin * (m0 * X.s[bi][0] + m1 * X.s[bi][1]);
+            acc[bi] = k4_chunk(acc[bi], d, dmin, sc0, m0, sc1, m1, al, ah, X.s[bi][0], X.s[bi][1]);
         }
     } else if constexpr (T == GGML_Q6_K) {
         const int i = c & 1;
@@ -246,16 +354,15 @@ __device__ __forceinline__ void dot_chunk(int c, const Raw<T> &r, const XF<T, B>
         }
 #pragma unroll
         for (int bi = 0; bi < B; ++bi) {
-            float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+            float a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                a0 = dot4u8(g0[u], &X.x[bi][4 * u], a0);
-                a1 = dot4u8(g1[u], &X.x[bi][16 + 4 * u], a1);
-                a2 = dot4u8(g2[u], &X.x[bi][32 + 4 * u], a2);
-                a3 = dot4u8(g3[u], &X.x[bi][48 + 4 * u], a3);
+                a[0] = dot4u8(g0[u], &X.x[bi][4 * u], a[0]);
+                a[1] = dot4u8(g1[u], &X.x[bi][16 + 4 * u], a[1]);
+                a[2] = dot4u8(g2[u], &X.x[bi][32 + 4 * u], a[2]);
+                a[3] = dot4u8(g3[u], &X.x[bi][48 + 4 * u], a[3]);
             }
-            acc[bi] += d * (sc[0] * (a0 - 32.f * X.s[bi][0]) + sc[1] * (a1 - 32.f * X.s[bi][1]) +
-                            sc[2] * (a2 - 32.f * X.s[bi][2]) + sc[3] * (a3 - 32.f * X.s[bi][3]));
+            acc[bi] = q6_chunk(acc[bi], d, sc, a, X.s[bi]);
         }
     } else if constexpr (T == GGML_Q8_0) {
         const float d = h2f(r.e0);

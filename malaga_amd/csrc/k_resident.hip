@@ -12,9 +12,14 @@
 // fence, counter or barrier between workgroups is needed, and every vector of every layer
 // has words of its own, so nothing is overwritten within a launch.  1024 words from 128
 // workgroups to 128 workgroups take 1.5 us including the workgroup's own reduction (256
-// workgroups: 2.0 us, so 128 share the rows).  A layer of the 600M model takes 17.5 us this
-// way (q4_K, 21 keys): seven hand-overs of 0.9 .. 1.5 us, three LayerNorms of 0.5, products
-// 4.5 and the two attentions 2.4 us; a sentence of 21 ids in and 18 tokens out 7.85 -> 5.47 ms.
+// workgroups: 2.0 us, so 128 share the rows).  A layer of the 600M model takes 18.1 us this
+// way (q4_K, 21 keys), most of it seven hand-overs of 0.9 .. 1.5 us.
+//
+// Results.  Every sum has the operations and the order of the per-layer launches of k_step.hip
+// (RowsK4, RowK6, Gather::norm, attn_half), so a step gives their bits, and which of the two a
+// call takes shows in its time only.  Orders of its own (16 values per lane, eight waves per
+// attention) took 17.4 us per layer, but then a call's tokens could differ with what other
+// threads had running: a sentence of 21 ids in and 18 tokens out 7.28 (per layer) / 4.95 / 5.12 ms.
 //
 // Roles.  Workgroups 0 .. H-1 own one attention head each: its self attention and, with the
 // head's 64 rows of the cross q projection, its cross attention.  The other kResPlain own
@@ -28,6 +33,7 @@
 // Every wait is bounded: a wave that runs out of polls (the workgroups are not all resident,
 // for instance behind other long kernels) raises *flag and goes on without waiting, so the
 // launch always ends; the caller sees the flag and decodes again with the other kernels.
+#include "attn_pair.hpp"
 #include "dequant.hpp"
 #include "gemv_core.hpp"
 #include "kernels.hpp"
@@ -111,13 +117,12 @@ struct Waiter {
 };
 
 // Vectors in LDS are kept as the lanes that multiply them read them, 16 bytes per lane and
-// instruction from 1 KB of whole rows of banks:
-//   q4_K / q5_K rows: d / 16 lanes of 16 values, lane 16 kb + 4 g + qt the bytes 8 qt .. 8 qt + 7
-//     of 64-value group g of block kb (low nibbles: x[256 kb + 64 g + 8 qt ..], high: + 32);
+// instruction from whole rows of banks:
+//   q4_K / q5_K rows: D / 32 lanes of one 32-value sub-block each (pos_k4);
 //   q6_K rows (FFN down): K / 64 lanes of 64 values, the chunks of load_chunk<q6_K>.
-__device__ __forceinline__ int pos_k4(int k, int lanes) {
-    const int lane = (k >> 6) * 4 + ((k >> 3) & 3), v = ((k >> 5) & 1) * 8 + (k & 7);
-    return (v >> 2) * (4 * lanes) + 4 * lane + (v & 3);
+template <int D>
+__device__ __forceinline__ int pos_k4(int k) {
+    return ((k & 31) >> 2) * (D / 8) + 4 * (k >> 5) + (k & 3);
 }
 __device__ __forceinline__ int pos_k6(int k, int lanes) {
     const int lane = (k >> 8) * 4 + ((k >> 7) & 1) * 2 + ((k >> 4) & 1), e = ((k >> 5) & 3) * 16 + (k & 15);
@@ -141,126 +146,132 @@ __device__ __forceinline__ uint2 ld8(gptr p) {
     const u32x2_t v = *reinterpret_cast<const __attribute__((address_space(1))) u32x2_t *>(p);
     return make_uint2(v.x, v.y);
 }
-__device__ __forceinline__ float ldf(gptr p) { return *reinterpret_cast<const __attribute__((address_space(1))) float *>(p); }
 
-// sum over aligned groups of W = 16, 32 or 64 lanes, in every lane
-template <int W>
-__device__ __forceinline__ float lanes_sum(float v) {
-    v += dpp_mov<kDppXor1>(v);
-    v += dpp_mov<kDppXor2>(v);
-    v += dpp_mov<kDppHalfMirror>(v);
-    v += dpp_mov<kDppMirror>(v);
-    if constexpr (W >= 32) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    }
-    if constexpr (W >= 64) {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    }
+constexpr int kDppPair0 = 0xA0, kDppPair1 = 0xF5;  // lane 2 i (2 i + 1) to both lanes of its pair
+
+// v[lane] + v[lane ^ 32]
+__device__ __forceinline__ float sum_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// v[lane] + v[lane ^ 16]
+__device__ __forceinline__ float sum_rows(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Sum over the 2^L2 chunks of a row whose value both lanes of a chunk's pair hold, in every
+// lane and in group_sum's order (a mirror within twice as many lanes meets the same chunks).
+template <int L2>
+__device__ __forceinline__ float sum_chunks(float v) {
+    if constexpr (L2 >= 1) v += dpp_mov<kDppXor2>(v);
+    if constexpr (L2 >= 2) v += dpp_mov<kDppHalfMirror>(v);
+    if constexpr (L2 >= 3) v += dpp_mov<kDppMirror>(v);
+    if constexpr (L2 >= 4) v = sum_rows(v);
     return v;
 }
 
-struct XK4 {  // a lane's 16 values and the sums of its two halves
-    float x[16], s[2];
-    __device__ __forceinline__ void load(const float *xs, int lanes, int lane) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 v = *reinterpret_cast<const float4 *>(xs + 4 * lanes * i + 4 * lane);
-            x[4 * i] = v.x, x[4 * i + 1] = v.y, x[4 * i + 2] = v.z, x[4 * i + 3] = v.w;
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const float *p = x + 8 * h;
-            s[h] = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-        }
-    }
-};
-
-// NP passes of 8 RPW rows (D / 16 = 2^LG lanes per row, RPW rows per wave) from row0 on, `rows`
-// in all.  A wave past the last row takes the last RPW rows (or all there are) again.
+// Rows of a q4_K / q5_K matrix, NP passes of 8 RPW rows: D / 32 lanes per row, one 32-value
+// sub-block each, RPW rows per wave.  The two lanes of a 64-value chunk hold 16 of its 32
+// packed bytes each and read the other's by DPP; lane 2 c sums the low nibbles, lane 2 c + 1
+// the high ones, and both form the chunk's value (k4_chunk).  Every sum has the operations and
+// the order of dot_chunk and group_sum, one chunk per lane.
 template <int T, int NP, int D>
 struct RowsK4 {
-    static constexpr int LG = D == 1024 ? 6 : D == 512 ? 5 : 4, RPW = 64 >> LG, K = D;
+    static constexpr int LPR = D / 32, RPW = 64 / LPR, L2 = D == 1024 ? 4 : D == 512 ? 3 : 2;
     static constexpr int B = T == GGML_Q4_K ? 144 : 176;
-    uint4 h[NP];
-    uint2 q[NP], qh[NP];  // qh: q5_K's fifth bits
-    __device__ __forceinline__ static int first_row(int p, int rows, int wave) {
-        return min((p * kResWaves + wave) * RPW, max(rows - RPW, 0));
-    }
+    uint4 h[NP], q[NP], qh[T == GGML_Q5_K ? NP : 1];  // qh: q5_K's fifth bits
+    __device__ __forceinline__ static int row(int p, int wave, int lane) { return (p * kResWaves + wave) * RPW + lane / LPR; }
     __device__ __forceinline__ void load(const ResMat &mt, int row0, int rows, int wave, int lane) {
         __builtin_amdgcn_sched_barrier(0);  // the registers' last values have been used
-        const int cl = lane & ((1 << LG) - 1), g = (cl >> 2) & 3, qt = cl & 3, rb = (K >> 8) * B;
-        const uint32_t off = uint32_t(min(lane >> LG, rows - 1) * rb + (cl >> 4) * B), oq = off + (B - 128) + 32 * g + 8 * qt;
+        // q5_K: the offsets are formed again each time (kept over the layers, they spill)
+        if constexpr (T == GGML_Q5_K) asm volatile("" : "+v"(lane));
+        const int sb = lane & (LPR - 1), hi = sb & 1, g = (sb >> 1) & 3;
+        constexpr int rb = (D >> 8) * B;
         const gptr m0 = uniform(mt.q) + size_t(row0) * rb;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const gptr base = m0 + first_row(p, rows, wave) * rb;
-            h[p] = ld16(base + off);
-            q[p] = ld8(base + oq);
-            if constexpr (T == GGML_Q5_K) qh[p] = ld8(base + off + 16 + 8 * qt);
+            const uint32_t off = uint32_t(min(row(p, wave, lane), rows - 1) * rb + (sb >> 3) * B);
+            h[p] = ld16(m0 + off);
+            q[p] = ld16(m0 + (off + (B - 128) + 32 * g + 16 * hi));
+            if constexpr (T == GGML_Q5_K) qh[p] = ld16(m0 + (off + 16 + 16 * hi));
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    // h becomes (d sc0, d sc1, dmin m0, dmin m1) of the lane's two sub-blocks (q4_K: d sc1 / 16,
-    // whose quants run() leaves 16 times as large).  Done while the wave has nothing to wait
-    // for but its vector, so that the scales cost nothing once that is there.
+    // h.y becomes the chunk's 6-bit (scale, min) pairs (sc0, m0, sc1, m1), a byte each.  Done
+    // while the wave has nothing to wait for but its vector.
     __device__ __forceinline__ void prepare(int lane) {
-        const int g = ((lane & ((1 << LG) - 1)) >> 2) & 3, sh0 = 8 * ((2 * g) & 3), sh1 = sh0 + 8;
+        const int g = ((lane & (LPR - 1)) >> 1) & 3, sh0 = 8 * ((2 * g) & 3);
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const uint4 hd = h[p];
-            const float d = h2f(hd.x), dmin = h2f(hd.x >> 16);
-            auto decode = [&](int sh, float &sc, float &mn) {
-                const uint32_t B0 = hd.y >> sh, B1 = hd.z >> sh, B2 = hd.w >> sh;
-                sc = d * float(g >= 2 ? ((B2 & 15u) | ((B0 >> 2) & 48u)) : (B0 & 63u));
-                mn = dmin * float(g >= 2 ? (((B2 >> 4) & 15u) | ((B1 >> 2) & 48u)) : (B1 & 63u));
-            };
-            float sc0, m0, sc1, m1;
-            decode(sh0, sc0, m0);
-            decode(sh1, sc1, m1);
-            if constexpr (T == GGML_Q4_K) sc1 *= 0.0625f;
-            h[p] = make_uint4(__float_as_uint(sc0), __float_as_uint(sc1), __float_as_uint(m0), __float_as_uint(m1));
+            const uint32_t B0 = h[p].y >> sh0, B1 = h[p].z >> sh0, B2 = h[p].w >> sh0;
+            // two bytes each: the pair's scales and mins
+            const uint32_t sc = g >= 2 ? ((B2 & 0x0F0Fu) | ((B0 >> 2) & 0x3030u)) : (B0 & 0x3F3Fu);
+            const uint32_t mn = g >= 2 ? (((B2 >> 4) & 0x0F0Fu) | ((B1 >> 2) & 0x3030u)) : (B1 & 0x3F3Fu);
+            h[p].y = __builtin_amdgcn_perm(mn, sc, 0x05010400u);
         }
         // here, not where the values are used (behind the barrier)
 #pragma unroll
-        for (int p = 0; p < NP; ++p) asm volatile("" : "+v"(h[p].x), "+v"(h[p].y), "+v"(h[p].z), "+v"(h[p].w));
+        for (int p = 0; p < NP; ++p) asm volatile("" : "+v"(h[p].x), "+v"(h[p].y));
+    }
+    // the chunk's value of every pass
+    __device__ __forceinline__ void chunks(const float *xs, int lane, float (&v)[NP]) const {
+        const int sb = lane & (LPR - 1), hi = sb & 1, g = (sb >> 1) & 3;
+        const uint32_t mask = hi ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
+        float a[NP], s = 0.f;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) a[p] = 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const float4 xv = *reinterpret_cast<const float4 *>(xs + u * (D / 8) + 4 * sb);
+            const float x[4] = {xv.x, xv.y, xv.z, xv.w};
+            s += x[0], s += x[1], s += x[2], s += x[3];
+            uint32_t w[NP];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                const uint32_t wo = (&q[p].x)[u & 3];
+                w[p] = u < 4 ? dpp_mov<kDppPair0>(wo) : dpp_mov<kDppPair1>(wo);
+                if constexpr (T == GGML_Q4_K) {
+                    w[p] &= mask;  // high: 16 * nibble, scaled back below
+                } else {
+                    const uint32_t ho = (&qh[p].x)[u & 3], hb = u < 4 ? dpp_mov<kDppPair0>(ho) : dpp_mov<kDppPair1>(ho);
+                    w[p] = ((w[p] >> (4 * hi)) & 0x0F0F0F0Fu) | (((hb >> (2 * g + hi)) & 0x01010101u) << 4);
+                }
+            }
+            dot4u8_items(w, x, a);
+        }
+        const float s0 = dpp_mov<kDppPair0>(s), s1 = dpp_mov<kDppPair1>(s);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            if constexpr (T == GGML_Q4_K) a[p] *= hi ? 0.0625f : 1.f;
+            const uint32_t sm = h[p].y;
+            v[p] = k4_chunk(0.f, h2f(h[p].x), h2f(h[p].x >> 16), ub0(sm), ub1(sm), ub2(sm), ub3(sm),
+                            dpp_mov<kDppPair0>(a[p]), dpp_mov<kDppPair1>(a[p]), s0, s1);
+        }
     }
     // store(row of the job, sum) by the first lane of each row
     template <class F>
     __device__ __forceinline__ void run(const float *xs, int rows, int wave, int lane, F &&store) const {
-        const int cl = lane & ((1 << LG) - 1), g = (cl >> 2) & 3;
-        XK4 X;
-        X.load(xs, 1 << LG, cl);
         float v[NP];
+        chunks(xs, lane, v);
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            uint2 qp = q[p];
-            // pass p starts when pass p - 2 has its sum: all of them expanded at once exceed
-            // the registers
-            if (p >= 2) asm volatile("" : "+v"(qp.x), "+v"(qp.y), "+v"(v[p - 2]));
-            float al[2], ah[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const uint32_t w = u ? qp.y : qp.x;
-                uint32_t lo = w & 0x0F0F0F0Fu, hi = w & 0xF0F0F0F0u;  // hi: 16 * nibble
-                if constexpr (T == GGML_Q5_K) {
-                    const uint32_t hb = u ? qh[p].y : qh[p].x;
-                    lo |= ((hb >> (2 * g)) & 0x01010101u) << 4;
-                    hi = ((w >> 4) & 0x0F0F0F0Fu) | (((hb >> (2 * g + 1)) & 0x01010101u) << 4);
-                }
-                al[u] = dot4u8(lo, X.x + 4 * u, 0.f);
-                ah[u] = dot4u8(hi, X.x + 8 + 4 * u, 0.f);
-            }
-            const float m = fmaf(__uint_as_float(h[p].z), X.s[0], __uint_as_float(h[p].w) * X.s[1]);
-            v[p] = fmaf(__uint_as_float(h[p].x), al[0] + al[1], __uint_as_float(h[p].y) * (ah[0] + ah[1])) - m;
+            const float r = sum_chunks<L2>(v[p]);
+            const int at = row(p, wave, lane);
+            if ((lane & (LPR - 1)) == 0 && at < rows) store(at, r);
         }
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            v[p] = lanes_sum<(1 << LG)>(v[p]);
-            if ((p * kResWaves + wave) * RPW < rows && cl == 0 && (lane >> LG) < rows)
-                store(first_row(p, rows, wave) + (lane >> LG), v[p]);
-        }
+    }
+    // the out-projections: a row's sums over the chunks of each head group of step_attn_head
+    // (head_geometry: D / 64 heads of one chunk in at most 8 groups) to out[row 8 + group]
+    static constexpr int GL2 = D == 1024 ? 1 : 0, kParts = (D / 64) >> GL2;
+    static_assert(kParts <= 8, "a row's partial sums take 8 floats");
+    __device__ __forceinline__ void run_parts(const float *xs, int rows, int wave, int lane, float *out) const {
+        static_assert(NP == 1, "one pass");
+        float v[1];
+        chunks(xs, lane, v);
+        const float r = sum_chunks<GL2>(v[0]);
+        const int at = row(0, wave, lane), sb = lane & (LPR - 1);
+        if ((sb & ((2 << GL2) - 1)) == 0 && at < rows) out[8 * at + (sb >> (1 + GL2))] = r;
     }
 };
 
@@ -297,101 +308,27 @@ struct RowK6 {
                                     ((A[u] >> 4) & 0x0F0F0F0Fu) | (H[u] & 0x30303030u),
                                     ((B[u] >> 4) & 0x0F0F0F0Fu) | ((H[u] >> 2) & 0x30303030u)};
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
+            for (int k = 0; k < 4; ++k) {  // sums in the order of gemv_load_x and dot_chunk
                 const float4 v = *reinterpret_cast<const float4 *>(xs + 4 * lanes * (4 * k + u) + o);
                 const float x[4] = {v.x, v.y, v.z, v.w};
                 q[k] = dot4u8(w4[k], x, q[k]);
-                sx[k] += (v.x + v.y) + (v.z + v.w);
+                sx[k] += x[0], sx[k] += x[1], sx[k] += x[2], sx[k] += x[3];
             }
         }
-        float acc = h2f(w.c.x) * (sc[0] * (q[0] - 32.f * sx[0]) + sc[1] * (q[1] - 32.f * sx[1]) +
-                                  sc[2] * (q[2] - 32.f * sx[2]) + sc[3] * (q[3] - 32.f * sx[3]));
+        float acc = q6_chunk(0.f, h2f(w.c.x), sc, q, sx);
         if (lane >= lanes) acc = 0.f;
-        return lanes_sum<64>(acc);
+        acc = sum_rows(group_sum<16>(acc));
+        return sum_halves(acc);
     }
 };
-
-// K and V of one key, 8 dimensions per lane
-struct KeyRegs {
-    uint4 k, v;
-};
-// sum over the lanes that share lane % 8
-__device__ __forceinline__ float sum_splits(float v) {
-    v += dpp_mov<0x128>(v);  // row_ror:8
-    const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
-    const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
-}
-
-// Attention of one query over n keys by the 8 waves of a workgroup: wave w takes keys
-// 64 c + 8 w + split, an online softmax per wave, its partial (64 sums, max, weight sum) to
-// slot w.  key(j): K and V of key j (the first round's are passed in).
-template <class KeyF>
-__device__ __forceinline__ void attn_partial(int n, int wave, int lane, const float *q, KeyRegs kv, KeyF &&key,
-                                             float *slot) {
-    const int sub = lane & 7, split = lane >> 3;
-    const float4 qa = *reinterpret_cast<const float4 *>(q + 8 * sub), qb = *reinterpret_cast<const float4 *>(q + 8 * sub + 4);
-    float m = -INFINITY, l = 0.f;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int j0 = 8 * wave; j0 < n; j0 += 8 * kResWaves) {  // wave-uniform
-        if (j0 != 8 * wave) kv = key(min(j0 + split, n - 1));
-        float s = h2f(kv.k.x) * qa.x;
-        s = fmaf(h2f(kv.k.x >> 16), qa.y, s);
-        s = fmaf(h2f(kv.k.y), qa.z, s);
-        s = fmaf(h2f(kv.k.y >> 16), qa.w, s);
-        s = fmaf(h2f(kv.k.z), qb.x, s);
-        s = fmaf(h2f(kv.k.z >> 16), qb.y, s);
-        s = fmaf(h2f(kv.k.w), qb.z, s);
-        s = fmaf(h2f(kv.k.w >> 16), qb.w, s);
-        s = group_sum<8>(s);
-        const bool in = j0 + split < n;
-        if (!in) s = -INFINITY;
-        const float mnew = fmaxf(m, wave_max(s));  // finite: key j0 is valid
-        const float r = expf(m - mnew), p = in ? expf(s - mnew) : 0.f;
-        l = l * r + p;
-        const uint32_t vv[4] = {in ? kv.v.x : 0u, in ? kv.v.y : 0u, in ? kv.v.z : 0u, in ? kv.v.w : 0u};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            acc[2 * e] = fmaf(p, h2f(vv[e]), acc[2 * e] * r);
-            acc[2 * e + 1] = fmaf(p, h2f(vv[e] >> 16), acc[2 * e + 1] * r);
-        }
-        m = mnew;
-    }
-    if (8 * wave < n) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] = sum_splits(acc[e]);
-        l = sum_splits(l);
-        if (split == 0) {
-            *reinterpret_cast<float4 *>(slot + 8 * sub) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-            *reinterpret_cast<float4 *>(slot + 8 * sub + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
-            if (sub == 0) slot[64] = m, slot[65] = l;
-        }
-    }
-}
-constexpr int kResSlot = 68;  // floats per partial
-__device__ __forceinline__ float attn_join(int n, int lane, const float *slots) {
-    const int nw = min(kResWaves, (n + 7) / 8);
-    float M = slots[64];
-    #pragma unroll
-    for (int w = 1; w < kResWaves; ++w) M = fmaxf(M, w < nw ? slots[w * kResSlot + 64] : M);
-    float o = 0.f, l = 0.f;
-#pragma unroll
-    for (int w = 0; w < kResWaves; ++w) {
-        if (w >= nw) break;
-        const float e = expf(slots[w * kResSlot + 64] - M);
-        l = fmaf(e, slots[w * kResSlot + 65], l);
-        o = fmaf(e, slots[w * kResSlot + lane], o);
-    }
-    return o / l;
-}
 
 constexpr int kResBias = (5 * kResMaxD + kResMaxD + kResMaxF) / kResPlain;  // >= kResHd
 
 struct ResLds {
     float h[kResMaxD], att[kResMaxD], catt[kResMaxD], u[kResMaxF];
     float res[64];  // a job's results on their way out
-    float qkv[3 * kResHd], q2[kResHd], slots[kResWaves * kResSlot];
+    float qkv[3 * kResHd], q2[kResHd];
+    float wsc[2 * 512], slots[2 * kHalfSlot];  // of the two waves of an attention (attn_half)
     float bias[kResMaxLayers][kResBias];  // this workgroup's rows: q k v | out | cross out | up | down, or cross q
     double red[2 * kResWaves];
     ResLayer layers[kResMaxLayers];
@@ -415,106 +352,144 @@ __device__ __forceinline__ void embed_row(const ResArgs &a, float *xs) {
     for (int j = 0; j < 16; ++j) xs[k0 + j] = e[j] * a.emb_scale + pr[j];
 }
 
-// The gathering threads' part of a d-wide vector: values t, t + 256, ..
+// float(1 / sqrt(v)) as the other step kernels round it: a correctly rounded square root and a
+// correctly rounded division in f64, then to f32.  Those two take 0.4 of the 0.9 us that a
+// LayerNorm would cost here, so: the hardware's estimate (2^-24) and a Newton step, whose
+// 2^-40 decides the rounding to f32 in all but one of some 10^4 cases.
+__device__ __forceinline__ float ln_rstd(double v) {
+    const double r0 = __builtin_amdgcn_rsq(v), r = r0 * fma(-0.5 * v * r0, r0, 1.5);
+    const float lo = float(r * (1.0 - 0x1p-40)), hi = float(r * (1.0 + 0x1p-40));
+    return lo == hi ? lo : float(1.0 / sqrt(v));
+}
+
+// The gathering threads' part of a D-wide vector: values at(0 .. 3) of the threads t < D / 4
+// (whole waves; a wave's 256 values in 64-value runs, as they are polled).
 template <int D>
 struct Gather {
-    static constexpr int N = D / kResGather;
+    static constexpr int N = 4;
     int t;
+    bool on;  // wave-uniform
     float x[N];  // the residual stream
-    __device__ __forceinline__ Gather(int t, const float *x0) : t(t) {
+    __device__ __forceinline__ int at(int k) const { return 4 * (t & ~63) + 64 * k + (t & 63); }
+    __device__ __forceinline__ Gather(int t, const float *x0) : t(t), on(t < D / 4) {
 #pragma unroll
-        for (int k = 0; k < N; ++k) x[k] = x0[t + k * kResGather];
+        for (int k = 0; k < N; ++k) x[k] = x0[on ? at(k) : 0];
     }
-    __device__ __forceinline__ void vec(const float *p, float (&v)[N]) const {
-        const gptr u = uniform(p);
-#pragma unroll
-        for (int k = 0; k < N; ++k) v[k] = ldf(u + uint32_t(4 * (t + k * kResGather)));
+    // values 4 t .. 4 t + 3
+    __device__ __forceinline__ float4 vec(const float *p) const {
+        const u32x4_t v = *reinterpret_cast<const __attribute__((address_space(1))) u32x4_t *>(
+            uniform(p) + uint32_t(on ? 16 * t : 0));
+        return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
     }
     __device__ __forceinline__ void add(Waiter &wt, const word_t *p) {
+        if (!on) return;
         float v[N];
-        wt.get<N>(p + t, kResGather, v);
+        wt.get<N>(p + at(0), 64, v);
 #pragma unroll
         for (int k = 0; k < N; ++k) x[k] += v[k];
     }
     __device__ __forceinline__ void gather(Waiter &wt, const word_t *p, float *xs) const {
+        if (!on) return;
         float v[N];
-        wt.get<N>(p + t, kResGather, v);
+        wt.get<N>(p + at(0), 64, v);
 #pragma unroll
-        for (int k = 0; k < N; ++k) xs[pos_k4(t + k * kResGather, D / 16)] = v[k];
+        for (int k = 0; k < N; ++k) xs[pos_k4<D>(at(k))] = v[k];
     }
-    // LayerNorm(x) into xs: two barriers of the workgroup.  Statistics in f64 as the other step
-    // kernels; d is a power of two (1 / d exact); 1 / sqrt as the hardware's estimate and a
-    // Newton step in f64, then rounded to f32 (a division and a square root in f64 took 0.4 us
-    // of the 0.9 a LayerNorm cost here).
-    __device__ __forceinline__ void norm(const float (&g)[N], const float (&b)[N], float eps, double *red, float *xs) const {
+    // LayerNorm(x) into xs: two barriers of the workgroup.  Statistics in f64 with the sums and
+    // the order of ln_to_lds (thread t sums values 4 t .. 4 t + 3, which it reads back from xs,
+    // then the wave, then the waves); D is a power of two, so 1 / D is exact.
+    __device__ __forceinline__ void norm(const float4 &g, const float4 &b, float eps, double *red, float *xs) const {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         double s1 = 0.0, s2 = 0.0;
+        if (on) {
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-            const double v = x[k];
-            s1 += v;
-            s2 += v * v;
+            for (int k = 0; k < N; ++k) xs[at(k)] = x[k];
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // this wave's LDS writes are done
+            __builtin_amdgcn_wave_barrier();
+            v = ld4(xs, t);
+            ln_acc(v, s1, s2);
         }
         s1 = wave_sum_f64(s1);
         s2 = wave_sum_f64(s2);
-        if ((t & 63) == 0) red[2 * (t >> 6)] = s1, red[2 * (t >> 6) + 1] = s2;
+        if ((t & 63) == 0) red[t >> 6] = s1, red[kResGatherWaves + (t >> 6)] = s2;
         lds_barrier();
-        s1 = s2 = 0.0;
-#pragma unroll
-        for (int k = 0; k < kResGatherWaves; ++k) s1 += red[2 * k], s2 += red[2 * k + 1];
+        s1 = (red[0] + red[1]) + (red[2] + red[3]);
+        s2 = (red[4] + red[5]) + (red[6] + red[7]);
         constexpr double inv = 1.0 / D;
-        const double mean = s1 * inv, v = fmax(s2 * inv - mean * mean, 0.0) + double(eps), r0 = __builtin_amdgcn_rsq(v);
-        const float rstd = float(r0 * fma(-0.5 * v * r0, r0, 1.5)), mu = float(mean);
-#pragma unroll
-        for (int k = 0; k < N; ++k) xs[pos_k4(t + k * kResGather, D / 16)] = (x[k] - mu) * rstd * g[k] + b[k];
+        const double mean = s1 * inv, ms = s2 * inv, var = fmax(fma(-mean, mean, ms), 0.0);
+        const float rstd = ln_rstd(var + double(eps)), mu = float(mean);
+        if (on) *reinterpret_cast<float4 *>(xs + pos_k4<D>(4 * t)) = ln_apply(v, mu, rstd, g, b);
         lds_barrier();
     }
 };
+static_assert(kResGatherWaves == 4, "norm adds four waves' sums");
 
 // waves 0..7 of a head's workgroup; six barriers per layer, as head_gather
 template <int T, int D>
 __device__ __forceinline__ void head_dot(const ResArgs &a, ResLds &s, uint32_t tag) {
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), hd = kResHd;
     const int h = blockIdx.x, cur = int(*a.step), ns = cur + 1, nc = int(a.lens[0]);
-    const int sub = lane & 7, j1 = 8 * wave + (lane >> 3);  // this lane's key of the first round
-    auto load_key = [&](const __half *k, const __half *v, int j) {
-        const size_t o = size_t(j) * hd + 8 * sub;
-        return KeyRegs{*reinterpret_cast<const uint4 *>(k + o), *reinterpret_cast<const uint4 *>(v + o)};
+    const int sub = lane & 7, split = lane >> 3;
+    // waves 0, 1 attend to the self cache, waves 2, 3 to the cross K/V (attn_half's two waves):
+    // each keeps one attention's first chunk, requested a layer ahead (it depends on nothing)
+    const bool self = wave < 2, cross = wave == 2 || wave == 3;
+    const int q = wave & 1;
+    uint4 kr[kHalfU], vr[kHalfU];
+    auto load_keys = [&](int l, int c) {
+        const int L = self ? a.m : a.s;
+        const __half *k = self ? a.kv + 2 * size_t(l) * a.self_pair + size_t(h) * a.m * hd
+                               : a.ckv + 2 * size_t(l) * a.cross_pair + size_t(h) * a.s * hd;
+        const gptr K = uniform(k), V = uniform(k + (self ? a.self_pair : a.cross_pair));
+#pragma unroll
+        for (int u = 0; u < kHalfU; ++u) {
+            const uint32_t o = uint32_t(min(half_key(8, c, u, q) + split, L - 1)) * uint32_t(2 * hd) + uint32_t(16 * sub);
+            kr[u] = ld16(K + o);
+            vr[u] = ld16(V + o);
+        }
     };
-    auto self_k = [&](int l) { return a.kv + 2 * size_t(l) * a.self_pair + size_t(h) * a.m * hd; };
-    auto cross_k = [&](int l) { return a.ckv + 2 * size_t(l) * a.cross_pair + size_t(h) * a.s * hd; };
-    RowsK4<T, D == 1024 ? 8 : D == 512 ? 4 : 2, D> cq;  // the head's 64 rows of the cross q projection
+    RowsK4<T, D == 1024 ? 4 : D == 512 ? 2 : 1, D> cq;  // the head's 64 rows of the cross q projection
     cq.load(s.layers[0].cq, h * hd, hd, wave, lane);
-    // the keys of a layer's first rounds depend on nothing: requested a layer ahead
-    KeyRegs sk = load_key(self_k(0), self_k(0) + a.self_pair, min(j1, a.m - 1)),
-            ck = load_key(cross_k(0), cross_k(0) + a.cross_pair, min(j1, a.s - 1));
+    if (self || cross) load_keys(0, 0);
     const __half *now = reinterpret_cast<const __half *>(s.qkv + hd);  // this step's k, v
+    float *wsc = s.wsc + q * 512, *slot = s.slots + q * kHalfSlot;
+    auto attend = [&](int l, int n, const float *qv, auto &&fix) {
+        const float4 qa = *reinterpret_cast<const float4 *>(qv + 8 * sub), qb = *reinterpret_cast<const float4 *>(qv + 8 * sub + 4);
+        fix(0);
+        attn_half<kResHd>(n, q, qa, qb, kr, vr, [&](int c) {
+            load_keys(l, c);
+            fix(c);
+        }, wsc, slot);
+    };
+    auto publish = [&](word_t *p) {
+        attn_combine2<kResHd>(s.slots, s.slots + kHalfSlot, s.res);
+        put(p + h * hd + lane, s.res[lane], tag);
+    };
     for (int l = 0; l < a.L; ++l) {
         const Words w = words_of(a, l);
         const int ln = min(l + 1, a.L - 1);
-        const __half *K = self_k(l), *V = K + a.self_pair, *CK = cross_k(l), *CV = CK + a.cross_pair;
-        float *slot = s.slots + wave * kResSlot;
         cq.prepare(lane);
         lds_barrier();  // q, k, v
-        auto self_key = [&](int j, KeyRegs r) {
-            if (j == cur) {
-                r.k = *reinterpret_cast<const uint4 *>(now + 8 * sub);
-                r.v = *reinterpret_cast<const uint4 *>(now + hd + 8 * sub);
-            }
-            return r;
-        };
-        attn_partial(ns, wave, lane, s.qkv, self_key(j1, sk),
-                     [&](int j) { return self_key(j, load_key(K, V, min(j, a.m - 1))); }, slot);
+        if (self)
+            attend(l, ns, s.qkv, [&](int c) {
+                // the cache's slot of this step is being written: its key comes from LDS
+#pragma unroll
+                for (int u = 0; u < kHalfU; ++u)
+                    if (half_key(8, c, u, q) + split == cur) {
+                        kr[u] = *reinterpret_cast<const uint4 *>(now + 8 * sub);
+                        vr[u] = *reinterpret_cast<const uint4 *>(now + hd + 8 * sub);
+                    }
+            });
         lds_barrier();
-        if (wave == 0) put(w.att + h * hd + lane, attn_join(ns, lane, s.slots), tag);
-        sk = load_key(self_k(ln), self_k(ln) + a.self_pair, min(j1, a.m - 1));
+        if (wave == 0) publish(w.att);
+        if (self) load_keys(ln, 0);
         lds_barrier();
         lds_barrier();  // LayerNorm(x)
         cq.run(s.h, hd, wave, lane, [&](int r, float v) { s.q2[r] = v + s.bias[l][r]; });
         lds_barrier();
-        attn_partial(nc, wave, lane, s.q2, ck, [&](int j) { return load_key(CK, CV, min(j, a.s - 1)); }, slot);
+        if (cross) attend(l, nc, s.q2, [](int) {});
         lds_barrier();
-        if (wave == 0) put(w.catt + h * hd + lane, attn_join(nc, lane, s.slots), tag);
-        ck = load_key(cross_k(ln), cross_k(ln) + a.cross_pair, min(j1, a.s - 1));
+        if (wave == 2) publish(w.catt);
+        if (cross) load_keys(ln, 0);
         cq.load(s.layers[ln].cq, h * hd, hd, wave, lane);
     }
 }
@@ -525,9 +500,7 @@ __device__ __forceinline__ void head_gather(const ResArgs &a, ResLds &s, Waiter 
     constexpr int hd = kResHd;
     const int t = int(threadIdx.x) - 64 * kResWaves, h = blockIdx.x, cur = int(*a.step);
     Gather<D> gt(t, s.u);
-    float g[Gather<D>::N], b[Gather<D>::N];
-    gt.vec(s.layers[0].cross_norm.g, g);
-    gt.vec(s.layers[0].cross_norm.b, b);
+    float4 g = gt.vec(s.layers[0].cross_norm.g), b = gt.vec(s.layers[0].cross_norm.b);
     for (int l = 0; l < a.L; ++l) {
         const Words w = words_of(a, l);
         if (t < 3 * hd) {  // whole waves: this head's q, k, v of the step
@@ -551,8 +524,8 @@ __device__ __forceinline__ void head_gather(const ResArgs &a, ResLds &s, Waiter 
         }
         gt.add(wt, w.out);
         gt.norm(g, b, a.eps, s.red, s.h);
-        gt.vec(s.layers[min(l + 1, a.L - 1)].cross_norm.g, g);
-        gt.vec(s.layers[min(l + 1, a.L - 1)].cross_norm.b, b);
+        g = gt.vec(s.layers[min(l + 1, a.L - 1)].cross_norm.g);
+        b = gt.vec(s.layers[min(l + 1, a.L - 1)].cross_norm.b);
         lds_barrier();
         lds_barrier();
     }
@@ -564,9 +537,9 @@ __device__ __forceinline__ void plain_dot(const ResArgs &a, ResLds &s) {
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int g = blockIdx.x - a.H, f = a.f, ru = f / kResPlain;
     constexpr int rd = D / kResPlain, rq = 3 * rd;
-    RowsK4<T, D == 1024 ? 3 : 1, D> qkv;
+    RowsK4<T, D == 1024 ? 2 : 1, D> qkv;
     RowsK4<T, 1, D> out, cout;
-    RowsK4<T, D == 1024 ? 4 : D == 512 ? 2 : 1, D> up;
+    RowsK4<T, D == 1024 ? 2 : 1, D> up;
     RowK6 down;
     auto load_qkv = [&](const ResLayer &y) { qkv.load(y.qkv, g * rq, rq, wave, lane); };
     auto load_out = [&](const ResLayer &y) { out.load(y.out, g * rd, rd, wave, lane); };
@@ -587,19 +560,17 @@ __device__ __forceinline__ void plain_dot(const ResArgs &a, ResLds &s) {
         qkv.run(s.h, rq, wave, lane, [&](int r, float v) { s.res[r] = v + bias[r]; });
         lds_barrier();
         load_qkv(nx);
-        bias += rq;
         out.prepare(lane);
         lds_barrier();
-        out.run(s.att, rd, wave, lane, [&](int r, float v) { s.res[r] = v + bias[r]; });
+        out.run_parts(s.att, rd, wave, lane, s.res);
         lds_barrier();
         load_out(nx);
-        bias += rd;
         cout.prepare(lane);
         lds_barrier();
-        cout.run(s.catt, rd, wave, lane, [&](int r, float v) { s.res[r] = v + bias[r]; });
+        cout.run_parts(s.catt, rd, wave, lane, s.res);
         lds_barrier();
         load_cout(nx);
-        bias += rd;
+        bias += rq + 2 * rd;
         up.prepare(lane);
         lds_barrier();
         lds_barrier();
@@ -618,7 +589,7 @@ __device__ __forceinline__ void plain_dot(const ResArgs &a, ResLds &s) {
 }
 
 // waves 8..11 of a projection workgroup
-template <int D>
+template <int T, int D>
 __device__ __forceinline__ void plain_gather(const ResArgs &a, ResLds &s, Waiter wt) {
     constexpr int NU = kResMaxF / kResGather;
     const int t = int(threadIdx.x) - 64 * kResWaves, f = a.f, g = blockIdx.x - a.H, ru = f / kResPlain;
@@ -629,27 +600,36 @@ __device__ __forceinline__ void plain_gather(const ResArgs &a, ResLds &s, Waiter
         lds_barrier();
         if (t < n) put(p + g * n + t, s.res[t], wt.tag);
     };
+    // the same for an out-projection, whose rows are sums over the head groups in order
+    auto publish_parts = [&](word_t *p, const float *bias) {
+        lds_barrier();
+        if (t < rd) {
+            const float *r = s.res + 8 * t;
+            float v = r[0];
+#pragma unroll
+            for (int k = 1; k < RowsK4<T, 1, D>::kParts; ++k) v += r[k];
+            put(p + g * rd + t, v + bias[t], wt.tag);
+        }
+    };
     Gather<D> gt(t, s.u);
-    float g1[Gather<D>::N], b1[Gather<D>::N], g2[Gather<D>::N], b2[Gather<D>::N];
-    gt.vec(s.layers[0].attn_norm.g, g1);
-    gt.vec(s.layers[0].attn_norm.b, b1);
+    float4 g1 = gt.vec(s.layers[0].attn_norm.g), b1 = gt.vec(s.layers[0].attn_norm.b), g2, b2;
     for (int l = 0; l < a.L; ++l) {
         const Words w = words_of(a, l);
         const ResLayer &ly = s.layers[l], &nx = s.layers[min(l + 1, a.L - 1)];
         if (l > 0) gt.add(wt, words_of(a, l - 1).down);
         gt.norm(g1, b1, a.eps, s.red, s.h);
         publish(w.q, rq);
-        gt.vec(ly.ffn_norm.g, g2);
-        gt.vec(ly.ffn_norm.b, b2);
-        gt.vec(nx.attn_norm.g, g1);
-        gt.vec(nx.attn_norm.b, b1);
+        g2 = gt.vec(ly.ffn_norm.g);
+        b2 = gt.vec(ly.ffn_norm.b);
+        g1 = gt.vec(nx.attn_norm.g);
+        b1 = gt.vec(nx.attn_norm.b);
         gt.gather(wt, w.att, s.att);
         lds_barrier();
-        publish(w.out, rd);
+        publish_parts(w.out, s.bias[l] + rq);
         gt.add(wt, w.out);  // arrives while the cross attention runs
         gt.gather(wt, w.catt, s.catt);
         lds_barrier();
-        publish(w.cout, rd);
+        publish_parts(w.cout, s.bias[l] + rq + rd);
         gt.add(wt, w.cout);
         gt.norm(g2, b2, a.eps, s.red, s.h);
         publish(w.u, ru);
@@ -671,7 +651,8 @@ __device__ __forceinline__ void plain_gather(const ResArgs &a, ResLds &s, Waiter
     }
     if (g == 0) {
 #pragma unroll
-        for (int k = 0; k < Gather<D>::N; ++k) a.x_out[t + k * kResGather] = gt.x[k];
+        for (int k = 0; k < Gather<D>::N; ++k)
+            if (gt.on) a.x_out[gt.at(k)] = gt.x[k];
         // every workgroup has published words of this launch, so all have read the epoch
         if (t == 0) *a.epoch = wt.tag + 1;
     }
@@ -713,7 +694,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(ResArgs a) {
         else plain_dot<T, D>(a, s);
     } else {
         if (head) head_gather<D>(a, s, wt);
-        else plain_gather<D>(a, s, wt);
+        else plain_gather<T, D>(a, s, wt);
     }
 }
 

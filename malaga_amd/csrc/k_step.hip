@@ -13,6 +13,7 @@
 // group's weights.  Workgroup 0 writes the updated residual stream to the other
 // half of a ping-pong pair.  Partial sums are added in a fixed order, so results
 // do not depend on scheduling.
+#include "attn_pair.hpp"
 #include "dequant.hpp"
 #include "gemv_core.hpp"
 #include "kernels.hpp"
@@ -299,88 +300,6 @@ struct HeadArgs {
 constexpr int kHeadCols = 256;  // max columns (HG * HD) per workgroup
 constexpr int kHeadParts = 8;   // head groups are sized so that P = H / HG <= this when possible
 
-// ---- one (row, head) pair shared by two waves (batch 1, head groups of <= 2 heads) ----
-// Wave q of the pair takes the SPL-key groups 2 i + q: pass u of its chunk c covers keys
-// SPL (2 (c U2 + u) + q) + split.  Each wave keeps an online softmax over its keys and
-// leaves its partial in LDS: po[HD] = sum_j p_j v_j (unnormalized), pml = (max, sum_j p_j)
-// with p_j = exp(s_j - max).  attn_combine2 then rescales the two partials to their common
-// max and divides: the same keys and the same order of sums whichever kernel runs it.
-constexpr int kHalfU = 4;                  // passes per chunk of a half
-constexpr int kHalfSlot = 128 + 2;         // floats of one wave's partial (HD <= 128)
-__host__ __device__ constexpr int half_key(int spl, int c, int u, int q) { return spl * (2 * (c * kHalfU + u) + q); }
-
-template <int HD, class LoadF>
-__device__ __forceinline__ void attn_half(int n, int q, const float4 &qa, const float4 &qb, const uint4 (&kr)[kHalfU],
-                                          const uint4 (&vr)[kHalfU], LoadF &&load, float *wsc, float *slot) {
-    constexpr int TPK = HD / 8, SPL = 64 / TPK;
-    const int lane = threadIdx.x & 63, sub = lane % TPK, split = lane / TPK;
-    float m = -INFINITY, l = 0.f;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int c = 0; half_key(SPL, c, 0, q) < n; ++c) {  // wave-uniform; chunk 0 is in flight
-        if (c) load(c);
-        float sc[kHalfU];
-        float cmax = -INFINITY;
-#pragma unroll
-        for (int u = 0; u < kHalfU; ++u) {
-            float s = h2f(kr[u].x) * qa.x;
-            s = fmaf(h2f(kr[u].x >> 16), qa.y, s);
-            s = fmaf(h2f(kr[u].y), qa.z, s);
-            s = fmaf(h2f(kr[u].y >> 16), qa.w, s);
-            s = fmaf(h2f(kr[u].z), qb.x, s);
-            s = fmaf(h2f(kr[u].z >> 16), qb.y, s);
-            s = fmaf(h2f(kr[u].w), qb.z, s);
-            s = fmaf(h2f(kr[u].w >> 16), qb.w, s);
-            s = group_sum<TPK>(s);
-            sc[u] = half_key(SPL, c, u, q) + split < n ? s : -INFINITY;
-            cmax = fmaxf(cmax, sc[u]);
-        }
-        const float mnew = fmaxf(m, wave_max(cmax));  // finite: the chunk's first key is valid
-        const float r = expf(m - mnew);
-        l *= r;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] *= r;
-#pragma unroll
-        for (int u = 0; u < kHalfU; ++u) {
-            const bool in = half_key(SPL, c, u, q) + split < n;
-            const float pj = in ? expf(sc[u] - mnew) : 0.f;
-            l += pj;
-            const uint32_t wv[4] = {in ? vr[u].x : 0u, in ? vr[u].y : 0u, in ? vr[u].z : 0u, in ? vr[u].w : 0u};
-#pragma unroll
-            for (int q2 = 0; q2 < 4; ++q2) {
-                acc[2 * q2] = fmaf(pj, h2f(wv[q2]), acc[2 * q2]);
-                acc[2 * q2 + 1] = fmaf(pj, h2f(wv[q2] >> 16), acc[2 * q2 + 1]);
-            }
-        }
-        m = mnew;
-    }
-    // every lane of a split holds that split's sum; count each split once
-    const float lsum = wave_sum(sub == 0 ? l : 0.f);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) wsc[lane * 8 + e] = acc[e];
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // this wave's LDS writes are done
-    __builtin_amdgcn_wave_barrier();
-    for (int e = lane; e < HD; e += 64) {
-        float o = 0.f;
-#pragma unroll
-        for (int s2 = 0; s2 < SPL; ++s2) o += wsc[(s2 * TPK + e / 8) * 8 + e % 8];
-        slot[e] = o;
-    }
-    if (lane == 0) {
-        slot[HD] = m;  // -inf when this wave had no key
-        slot[HD + 1] = lsum;
-    }
-}
-
-// out[e] of the pair from the partials of its two waves (after a workgroup barrier)
-template <int HD>
-__device__ __forceinline__ void attn_combine2(const float *s0, const float *s1, float *out) {
-    const int lane = threadIdx.x & 63;
-    const float m0 = s0[HD], m1 = s1[HD], M = fmaxf(m0, m1);  // m0 finite: wave 0 has key 0
-    const float e0 = expf(m0 - M), e1 = expf(m1 - M);
-    const float inv = 1.f / (e0 * s0[HD + 1] + e1 * s1[HD + 1]);
-    for (int e = lane; e < HD; e += 64) out[e] = (e0 * s0[e] + e1 * s1[e]) * inv;
-}
-
 // Workgroup (g, r): attention of heads [g HG, (g + 1) HG) for all nb rows, then
 // part[g][bi][row] = sum_{c < C} W[row][g C + c] * att[bi][g C + c] for the RW
 // rows [r RW, (r + 1) RW), one (row, chunk) item per thread.  Workgroups with the
@@ -586,66 +505,6 @@ __global__ __launch_bounds__(256) void k_attn_head(HeadArgs a) {
 constexpr int kXThreads = 512;  // 8 waves
 constexpr int kXItems = 4;      // (row, chunk) items of the q projection per thread
 
-// dot4u8 as one asm block: each byte is converted where it is used, so a schedule
-// cannot convert every item's bytes ahead of their products (which overflows the
-// registers of a multi-item dot); same operations, same order
-[[maybe_unused]] __device__ __forceinline__ float dot4u8_chain(uint32_t v, const float (&x)[4], float acc) {
-    float t0, t1, t2, t3;
-    asm("v_cvt_f32_ubyte0 %1, %5\n\t"
-        "v_cvt_f32_ubyte1 %2, %5\n\t"
-        "v_fmac_f32 %0, %1, %6\n\t"
-        "v_cvt_f32_ubyte2 %3, %5\n\t"
-        "v_fmac_f32 %0, %2, %7\n\t"
-        "v_cvt_f32_ubyte3 %4, %5\n\t"
-        "v_fmac_f32 %0, %3, %8\n\t"
-        "v_fmac_f32 %0, %4, %9"
-        : "+v"(acc), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
-        : "v"(v), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
-    return acc;
-}
-
-// dot4u8_chain of four items' words against the same four x values, as one asm block:
-// byte b of every word is converted, then the four products are added, so the four
-// items' dependent chains interleave (one chain per block left each product waiting for
-// the previous one); per item the operations and their order are dot4u8_chain's
-__device__ __forceinline__ void dot4u8_chain4(const uint32_t (&v)[4], const float (&x)[4], float (&acc)[4]) {
-    float t0, t1, t2, t3;
-    asm("v_cvt_f32_ubyte0 %4, %8\n\t"
-        "v_cvt_f32_ubyte0 %5, %9\n\t"
-        "v_cvt_f32_ubyte0 %6, %10\n\t"
-        "v_cvt_f32_ubyte0 %7, %11\n\t"
-        "v_fmac_f32 %0, %4, %12\n\t"
-        "v_fmac_f32 %1, %5, %12\n\t"
-        "v_fmac_f32 %2, %6, %12\n\t"
-        "v_fmac_f32 %3, %7, %12\n\t"
-        "v_cvt_f32_ubyte1 %4, %8\n\t"
-        "v_cvt_f32_ubyte1 %5, %9\n\t"
-        "v_cvt_f32_ubyte1 %6, %10\n\t"
-        "v_cvt_f32_ubyte1 %7, %11\n\t"
-        "v_fmac_f32 %0, %4, %13\n\t"
-        "v_fmac_f32 %1, %5, %13\n\t"
-        "v_fmac_f32 %2, %6, %13\n\t"
-        "v_fmac_f32 %3, %7, %13\n\t"
-        "v_cvt_f32_ubyte2 %4, %8\n\t"
-        "v_cvt_f32_ubyte2 %5, %9\n\t"
-        "v_cvt_f32_ubyte2 %6, %10\n\t"
-        "v_cvt_f32_ubyte2 %7, %11\n\t"
-        "v_fmac_f32 %0, %4, %14\n\t"
-        "v_fmac_f32 %1, %5, %14\n\t"
-        "v_fmac_f32 %2, %6, %14\n\t"
-        "v_fmac_f32 %3, %7, %14\n\t"
-        "v_cvt_f32_ubyte3 %4, %8\n\t"
-        "v_cvt_f32_ubyte3 %5, %9\n\t"
-        "v_cvt_f32_ubyte3 %6, %10\n\t"
-        "v_cvt_f32_ubyte3 %7, %11\n\t"
-        "v_fmac_f32 %0, %4, %15\n\t"
-        "v_fmac_f32 %1, %5, %15\n\t"
-        "v_fmac_f32 %2, %6, %15\n\t"
-        "v_fmac_f32 %3, %7, %15"
-        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
-        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
-}
-
 // group_sum_dyn of N values at once, step by step, so that their DPP chains interleave
 // (per value the same operations in the same order)
 template <int N>
@@ -701,16 +560,8 @@ __device__ __forceinline__ void dot_items(int c, const Raw<T> (&r)[KI], const fl
                 hi[k] = wu & 0xF0F0F0F0u;  // 16 * nibble; scaled back below
             }
         }
-        if constexpr (KI == 4) {
-            dot4u8_chain4(lo, vl, al);
-            dot4u8_chain4(hi, vh, ah);
-        } else {
-#pragma unroll
-            for (int k = 0; k < KI; ++k) {
-                al[k] = dot4u8_chain(lo[k], vl, al[k]);
-                ah[k] = dot4u8_chain(hi[k], vh, ah[k]);
-            }
-        }
+        dot4u8_items(lo, vl, al);
+        dot4u8_items(hi, vh, ah);
     }
     // the sums of gemv_load_x (xslot: values 0..31 -> 0, 32..63 -> 1), in its order
 #pragma unroll
@@ -734,9 +585,7 @@ __device__ __forceinline__ void dot_items(int c, const Raw<T> (&r)[KI], const fl
         const float d = h2f(r[k].h.x), dmin = h2f(r[k].h.x >> 16);
         float a0 = ah[k];
         if constexpr (T == GGML_Q4_K) a0 *= 0.0625f;
-        float acc = 0.f;
-        acc += d * (sc0 * al[k] + sc1 * a0) - dmin * (m0 * s0 + m1 * s1);
-        out[k] = acc;
+        out[k] = k4_chunk(0.f, d, dmin, sc0, m0, sc1, m1, al[k], a0, s0, s1);
     }
 }
 

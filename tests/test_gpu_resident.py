@@ -1,4 +1,5 @@
-"""The resident batch-1 decoder step (k_resident.hip): all layers in one launch."""
+"""The resident batch-1 decoder step (k_resident.hip): all layers in one launch, with the bits
+of the per-layer launches it stands in for."""
 import threading
 
 import numpy as np
@@ -53,40 +54,65 @@ def test_resident_step_matches_oracle(model, preset, d, f):
         gpu.close()
 
 
+def load(path, monkeypatch, **env):
+    """A translator that read these variables at load."""
+    with monkeypatch.context() as m:
+        for k, v in env.items():
+            m.setenv(k, v)
+        return M.Translator.load(path)
+
+
+@pytest.mark.parametrize("preset", ["q4_k_m", "q5_k_m"])
+@pytest.mark.parametrize("d,f", [(256, 512), (512, 1536), (1024, 4096), (1024, 2560)])
+def test_resident_step_equals_per_layer_launches(model, monkeypatch, preset, d, f):
+    """Tokens and winning logits bit for bit, with one key, keys on both sides of the attention's
+    groups of 8 and rounds of 64 in both attentions, and several rounds: the sums have one
+    order, so what a call returns does not depend on the launches it gets."""
+    path = model(preset, d, f)
+    on, off = load(path, monkeypatch), load(path, monkeypatch, MALAGA_RESIDENT_STEP="0")
+    try:
+        for n, new in ((1, 1), (8, 9), (9, 8), (63, 66), (64, 3), (65, 3), (130, 140), (200, 30)):
+            src = [np.random.default_rng(n * d).integers(4, 1200, n).tolist()]
+            a = on.greedy_top(on.encode_cross(src), 1100, new, eos_mask=True)
+            b = off.greedy_top(off.encode_cross(src), 1100, new, eos_mask=True)
+            assert a == b, (n, new)
+    finally:
+        on.close()
+        off.close()
+
+
 def test_resident_step_off_and_out_of_polls(model, monkeypatch):
     """MALAGA_RESIDENT_STEP=0 and a launch whose waits run out at once (the flag is raised and
-    the call decodes again per layer, then and from there on) give what the per-layer step
-    gives."""
+    the call decodes again per layer) give the same bits."""
     path = model("q4_k_m", 512, 1536)
     src = [np.random.default_rng(3).integers(4, 1200, 11).tolist()]
     out = {}
     for name, env in (("on", {}), ("off", {"MALAGA_RESIDENT_STEP": "0"}), ("stuck", {"MALAGA_RESIDENT_SPINS": "0"})):
-        with monkeypatch.context() as m:
-            for k, v in env.items():
-                m.setenv(k, v)
-            gpu = M.Translator.load(path)
+        gpu = load(path, monkeypatch, **env)
         batch = gpu.encode_cross(src)
         out[name] = [gpu.greedy_top(batch, 1100, 20, eos_mask=True) for _ in range(3)]
         gpu.close()
-    assert out["stuck"] == out["off"]
-    for (a, ta), (b, tb) in zip(out["on"], out["off"]):
-        assert a == b and np.abs(np.array(ta) - np.array(tb)).max() < 1e-3
+    assert out["stuck"] == out["off"] == out["on"]
 
 
 def test_resident_step_from_several_threads(model):
     """Contexts of their own on one device: one call at a time has the resident launch, the
-    others decode per layer meanwhile; every call gives its own sentence's tokens."""
+    others decode per layer meanwhile; every call gives the tokens and logits, to the bit, that
+    it gives alone."""
     path = model("q4_k_m", 256, 512)
     srcs = [[np.random.default_rng(50 + i).integers(4, 1200, 4 + 5 * i).tolist()] for i in range(3)]
+
+    def decode(t, src):
+        return t.greedy_top(t.encode_cross(src), 1100, 30, eos_mask=True)
+
     ref = M.Translator.load(path)
-    want = [ref.generate(s, 1100, M.GenOptions(max_new_tokens=30, eos_mask=True)) for s in srcs]
+    want = [decode(ref, s) for s in srcs]
     ref.close()
     ts = [M.Translator.load(path) for _ in srcs]
     done = []
 
     def work(i):
-        done.append((i, all(ts[i].generate(srcs[i], 1100, M.GenOptions(max_new_tokens=30, eos_mask=True)) == want[i]
-                            for _ in range(8))))
+        done.append((i, all(decode(ts[i], srcs[i]) == want[i] for _ in range(8))))
 
     threads = [threading.Thread(target=work, args=(i,)) for i in range(len(ts))]
     for t in threads:
