@@ -208,6 +208,13 @@ int mlg_server_stats(const mlg_server *s, int64_t *jobs, int64_t *groups, int64_
 /* GraphCache::clear (src/graph.rs:192-200). */
 void mlg_clear_graphs(mlg_model *m);
 int mlg_graph_stats(const mlg_model *m, int *entries, int *graphs, int *capture_enabled);
+/* The launch that runs every decoder layer of one sentence's greedy step at once: *active = 1 if
+   the next such call may take it (0: model or device not covered, switched off by
+   MALAGA_RESIDENT_STEP=0, or pausing after a launch whose waits ran out), the calls that it
+   decoded, and those decoded again per layer, with the same results, after such a launch. */
+int mlg_resident_stats(const mlg_model *m, int *active, int64_t *calls, int64_t *redone);
+/* Test hook: polls per wait of that launch from here on (0: its first wait runs out). */
+void mlg_debug_resident_spins(mlg_model *m, uint32_t polls);
 /* The cache's entries, least recently used first (the eviction order of src/graph.rs:301-323):
    up to cap rows of (batch bucket, source bucket, output bucket, has a graph) into keys
    [cap][4]; returns the number of entries (or a negative status).  Introspection for

@@ -273,6 +273,14 @@ class Translator:
         check(self.lib.mlg_graph_stats(self.h, C.byref(e), C.byref(g), C.byref(c)))
         return {"entries": e.value, "graphs": g.value, "capture": bool(c.value)}
 
+    def resident_stats(self) -> dict:
+        """Greedy decoding of one sentence by the launch that runs all decoder layers at once:
+        whether the next call may take it, the calls that it decoded, and those decoded again
+        per layer (the same results) after a launch whose waits ran out."""
+        a, n, r = C.c_int(), C.c_int64(), C.c_int64()
+        check(self.lib.mlg_resident_stats(self.h, C.byref(a), C.byref(n), C.byref(r)))
+        return {"active": bool(a.value), "calls": n.value, "redone": r.value}
+
 
 # ----------------------------------------------------------------- configs
 

@@ -106,6 +106,8 @@ SIGNATURES = {
                                    C.POINTER(C.c_int64)]),
     "mlg_clear_graphs": (None, [_P]),
     "mlg_graph_stats": (C.c_int, [_P, _intp, _intp, _intp]),
+    "mlg_resident_stats": (C.c_int, [_P, _intp, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
+    "mlg_debug_resident_spins": (None, [_P, C.c_uint32]),
     "mlg_graph_cache_keys": (C.c_int, [_P, _P, C.c_int]),
     "mlg_debug_fail_alloc_after": (None, [C.c_long]),
     "mlg_debug_tile_major": (C.c_int64, [C.c_uint32, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_int64]),

@@ -514,6 +514,15 @@ int mlg_graph_stats(const mlg_model *m, int *entries, int *graphs, int *capture_
     return MLG_OK;
 }
 
+int mlg_resident_stats(const mlg_model *m, int *active, int64_t *calls, int64_t *redone) {
+    if (!m || !active || !calls || !redone) return set_err(MLG_ERR_INVALID, "null argument");
+    std::lock_guard<std::mutex> lk(m->m->ctx->mu);
+    *active = m->m->resident_active() ? 1 : 0;
+    *calls = m->m->res_use.calls;
+    *redone = m->m->res_use.redone;
+    return MLG_OK;
+}
+
 int mlg_graph_cache_keys(const mlg_model *m, int *keys, int cap) {
     if (!m || cap < 0 || (cap && !keys)) return -set_err(MLG_ERR_INVALID, "bad argument");
     std::lock_guard<std::mutex> lk(m->m->ctx->mu);
@@ -525,6 +534,12 @@ int mlg_graph_cache_keys(const mlg_model *m, int *keys, int cap) {
         keys[4 * i + 3] = k[i].graph ? 1 : 0;
     }
     return int(k.size());
+}
+
+void mlg_debug_resident_spins(mlg_model *m, uint32_t polls) {
+    if (!m) return;
+    std::lock_guard<std::mutex> lk(m->m->ctx->mu);
+    m->m->set_resident_spins(polls);
 }
 
 void mlg_debug_fail_alloc_after(long n) { mlg::set_fail_alloc_after(n); }

@@ -530,7 +530,9 @@ void Model::load(const std::string &path) {
 
 // The layer table of the resident batch-1 step, where its kernel covers the model (one type
 // for all projections) and the device.  MALAGA_RESIDENT_STEP=0 keeps the per-layer launches;
-// MALAGA_RESIDENT_SPINS sets the polls per wait (a test hook; 2^20 are about a second).
+// MALAGA_RESIDENT_SPINS sets the polls per wait (a test hook).  The default, 2^16, is about
+// 60 ms: a step takes 0.2 ms alone, and a call that waits longer, for compute units that other
+// kernels hold, is decoded sooner by the per-layer launches.
 void Model::build_resident() {
     const char *off = std::getenv("MALAGA_RESIDENT_STEP");
     if (dec.empty() || no_fuse_ || split_cross_ || (off && std::string(off) == "0")) return;
@@ -554,8 +556,17 @@ void Model::build_resident() {
     owned_.push_back(t);
     check_hip(hipMemcpy(t, table.data(), table.size() * sizeof(ResLayer), hipMemcpyHostToDevice), "upload");
     const char *spins = std::getenv("MALAGA_RESIDENT_SPINS");
-    res_spins_ = spins ? uint32_t(std::strtoul(spins, nullptr, 10)) : 1u << 20;
+    res_spins_ = spins ? uint32_t(std::strtoul(spins, nullptr, 10)) : 1u << 16;
     res_layers_ = t;
+}
+
+// A launch that gave up leaves words of its tag and, from workgroups that started after its
+// end, of the next one: none may be there for another launch to take for its own.
+void Model::reset_resident(StaticState &st) {
+    const size_t words = step_resident_words(cfg.d_model, cfg.decoder_ffn, int(dec.size()));
+    check_hip(fill_u32(reinterpret_cast<uint32_t *>(st.words), 0, 2 * words, ctx->stream), "fill");
+    check_hip(fill_u32(st.epoch, 1, 1, ctx->stream), "fill");
+    check_hip(fill_u32(st.res_flag, 0, 1, ctx->stream), "fill");
 }
 
 bool Model::resident_ok(const DevMatrix &emb, int b, int m, int s) const {
@@ -802,15 +813,12 @@ std::unique_ptr<StaticState> Model::new_state(int b, int s, int m, bool logits, 
         st->part = static_cast<float *>(get(size_t(H) * b * d * 4, "attention partial sums"));
         st->part2 = static_cast<float *>(get(size_t(H) * b * d * 4, "cross attention partial sums"));
     }
-    st->resident = resident && st->fused;
-    if (st->resident) {
-        const size_t words = step_resident_words(d, cfg.decoder_ffn, L);
-        st->words = static_cast<uint64_t *>(get(words * sizeof(uint64_t), "resident step words"));
+    if (resident && st->fused) {
+        st->words = static_cast<uint64_t *>(get(step_resident_words(d, cfg.decoder_ffn, L) * sizeof(uint64_t),
+                                                "resident step words"));
         st->epoch = static_cast<uint32_t *>(get(4, "resident step epoch"));
         st->res_flag = static_cast<uint32_t *>(get(4, "resident step flag"));
-        check_hip(fill_u32(reinterpret_cast<uint32_t *>(st->words), 0, 2 * words, ctx->stream), "fill");
-        check_hip(fill_u32(st->epoch, 1, 1, ctx->stream), "fill");
-        check_hip(fill_u32(st->res_flag, 0, 1, ctx->stream), "fill");
+        reset_resident(*st);
     }
     if (!st->fused && dgemm_step_ok(b))
         st->lnstat = static_cast<double *>(get(size_t(d / 16) * b * 2 * sizeof(double), "LayerNorm statistics"));
@@ -1214,23 +1222,32 @@ GraphCache::~GraphCache() {
     if (fin_ev_) (void)hipEventDestroy(fin_ev_);
 }
 
-size_t GraphCache::Entry::bytes() const { return st->bytes + (exec ? kGraphBytes : 0); }
+size_t GraphCache::Entry::bytes() const { return st->bytes + graphs() * kGraphBytes; }
+
+bool GraphCache::Entry::drop_graphs() {
+    const bool any = graphs() > 0;
+    for (hipGraphExec_t &x : exec) {
+        if (x) (void)hipGraphExecDestroy(x);
+        x = nullptr;
+    }
+    return any;
+}
 
 size_t GraphCache::graphs() const {
     size_t n = 0;
-    for (auto &e : entries_) n += e.exec != nullptr;
+    for (auto &e : entries_) n += e.graphs();
     return n;
 }
 
 // src/graph.rs:193-200, 325-335: destroyed graphs' memory goes back to the driver
 void GraphCache::clear() {
-    bool had_graphs = false;
-    for (auto &e : entries_)
-        if (e.exec) {
-            (void)hipGraphExecDestroy(e.exec);
-            had_graphs = true;
-        }
+    drop_graphs();
     entries_.clear();
+}
+
+void GraphCache::drop_graphs() {
+    bool had_graphs = false;
+    for (auto &e : entries_) had_graphs |= e.drop_graphs();
     if (had_graphs) trim_graph_memory();
 }
 
@@ -1251,10 +1268,7 @@ void GraphCache::evict(const Entry *keep) {
         for (auto it = entries_.begin(); it != entries_.end(); ++it)
             if (&*it != keep && (victim == entries_.end() || it->last_used < victim->last_used)) victim = it;
         if (victim == entries_.end()) break;
-        if (victim->exec) {
-            (void)hipGraphExecDestroy(victim->exec);
-            dropped_graph = true;
-        }
+        dropped_graph |= victim->drop_graphs();
         entries_.erase(victim);
     }
     if (dropped_graph) trim_graph_memory();
@@ -1266,7 +1280,7 @@ std::vector<GraphCache::Key> GraphCache::keys() const {
     std::stable_sort(order.begin(), order.end(),
                      [](const Entry *a, const Entry *b) { return a->last_used < b->last_used; });
     std::vector<Key> out;
-    for (const Entry *e : order) out.push_back(Key{e->b, e->s, e->m, e->exec != nullptr});
+    for (const Entry *e : order) out.push_back(Key{e->b, e->s, e->m, e->graphs() > 0});
     return out;
 }
 
@@ -1306,7 +1320,7 @@ struct ResidentTurn {
 
 std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tgt_lang, int max_new, int sync_every,
                                                    bool eos_mask, bool use_graph, const Shortlist *sl,
-                                                   std::vector<std::vector<float>> *top) {
+                                                   std::vector<std::vector<float>> *top, bool may_reside) {
     Model &m = *model_;
     if (!sl) m.ensure_embed();  // the full LM head and input embeddings
     hipStream_t s = m.ctx->stream;
@@ -1317,24 +1331,30 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     const int kb = b, ks = bucket(src.s, 16, max_m), km = bucket(max_new + 2, 32, max_m);
     ++clock_;
     ResidentTurn turn;  // until the stream is drained below
-    const bool resident = m.resident_ok(sl ? sl->head : m.embed, kb, km, ks) && turn.take(m.ctx->device);
+    const bool can = m.resident_ok(sl ? sl->head : m.embed, kb, km, ks);
+    bool resident = false;
+    if (can && may_reside) {
+        if (m.res_use.pause > 0) --m.res_use.pause;
+        else resident = turn.take(m.ctx->device);
+    }
     Entry *e = nullptr;
     for (auto &it : entries_)
-        if (it.b == kb && it.s == ks && it.m == km && it.sl == sl && it.resident == resident) e = &it;
+        if (it.b == kb && it.s == ks && it.m == km && it.sl == sl) e = &it;
     if (!e) {
         Entry ne;
         ne.b = kb;
         ne.s = ks;
         ne.m = km;
         ne.sl = sl;
-        ne.resident = resident;
-        ne.st = m.new_state(kb, ks, km, false, false, sl, false, resident);
+        ne.st = m.new_state(kb, ks, km, false, false, sl, false, can);
         entries_.push_back(std::move(ne));
         e = &entries_.back();
         evict(e);
     }
     e->last_used = clock_;
     StaticState &st = *e->st;
+    st.resident = resident;
+    hipGraphExec_t &step_graph = e->exec[resident];
     const int mask_id = eos_mask ? c.eos_token_id : -1;
 
     std::vector<uint32_t> rows(static_cast<size_t>(n));
@@ -1342,9 +1362,9 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     // step 0 consumes decoder_start; its token is replaced by the forced target language.
     // Once the bucket's graph exists these two steps replay it as well (the graph is the
     // same step; the fill and the flag reset between them are ordinary stream work).
-    const bool replay = capture && e->exec;
+    const bool replay = capture && step_graph;
     auto one_step = [&] {
-        if (replay) check_hip(hipGraphLaunch(e->exec, s), "graph launch");
+        if (replay) check_hip(hipGraphLaunch(step_graph, s), "graph launch");
         else m.step(st, true, mask_id);
     };
     m.reset_state(st, src, rows, uint32_t(c.decoder_start_token_id));
@@ -1358,7 +1378,7 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     int steps = 2;
     const int max_steps = std::min(max_new + 1, st.m);
 
-    if (capture && !e->exec && steps < max_steps) {
+    if (capture && !step_graph && steps < max_steps) {
         check_hip(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
         hipGraph_t graph = nullptr;
         try {
@@ -1373,7 +1393,7 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
         const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         check_hip(ie, "graph instantiate");
-        e->exec = exec;
+        step_graph = exec;
     }
     if (fin_cap_ < size_t(st.b)) {
         if (fin_host_) (void)hipHostFree(fin_host_);
@@ -1401,7 +1421,7 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
             check_hip(hipEventRecord(fin_ev_, s), "event");
             pending = true;
         }
-        if (capture && e->exec) check_hip(hipGraphLaunch(e->exec, s), "graph launch");
+        if (capture && step_graph) check_hip(hipGraphLaunch(step_graph, s), "graph launch");
         else m.step(st, true, mask_id);
         ++steps;
     }
@@ -1414,11 +1434,12 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     uint32_t stuck = 0;
     if (st.resident) check_hip(hipMemcpyAsync(&stuck, st.res_flag, 4, hipMemcpyDeviceToHost, s), "D2H");
     check_hip(hipStreamSynchronize(s), "sync");
-    if (stuck) {  // the results are void; from here on this model launches per layer
-        m.drop_resident();
-        clear();
-        return run(src, tgt_lang, max_new, sync_every, eos_mask, use_graph, sl, top);
+    if (stuck) {  // the results are void
+        m.reset_resident(st);
+        m.res_use.failed();
+        return run(src, tgt_lang, max_new, sync_every, eos_mask, use_graph, sl, top, false);
     }
+    if (st.resident) m.res_use.succeeded();
     if (err) fail(ERR_INVALID, kNonFiniteLogits);
     std::vector<std::vector<uint32_t>> res(static_cast<size_t>(n));
     if (top) top->assign(static_cast<size_t>(n), {});

@@ -137,8 +137,9 @@ struct StaticState {
     uint8_t *src_q = nullptr;             // lazy embeddings: token_embd rows of src_ids (device layout)
     uint32_t *src_iota = nullptr;         // lazy embeddings: 0 .. b*s-1
     bool fused = false;                   // decoder step uses the fused kernels of k_step.hip
-    // batch-1 greedy: the layers run as one resident launch (k_resident.hip) over these words
-    // (with fused, whose kernels remain the way when that launch could not finish its waits)
+    // batch-1 greedy where the model is covered: buffers of the resident launch
+    // (k_resident.hip), and whether step() uses it now (else, bit for bit the same, the fused
+    // kernels)
     bool resident = false;
     uint64_t *words = nullptr;
     uint32_t *epoch = nullptr, *res_flag = nullptr;
@@ -163,6 +164,7 @@ class GraphCache {
     ~GraphCache();
     bool capture_enabled() const { return capture_; }
     void clear();
+    void drop_graphs();  // the states stay
     // Greedy decoding of an encoded batch; rows stripped at EOS (src/graph.rs:204-298).
     // sl: decode over the shortlist + source tokens (src/graph.rs:204-298 with a shortlist).
     // top (optional): receives each row's winning logits, one per returned token.
@@ -183,15 +185,16 @@ class GraphCache {
     struct Entry {
         int b, s, m;
         const Shortlist *sl = nullptr;  // part of the key (src/graph.rs:157)
-        bool resident = false;          // part of the key
         std::unique_ptr<StaticState> st;
-        hipGraphExec_t exec = nullptr;
+        hipGraphExec_t exec[2] = {nullptr, nullptr};  // step graph; [1]: with the resident launch
         uint64_t last_used = 0;
+        size_t graphs() const { return size_t(exec[0] != nullptr) + size_t(exec[1] != nullptr); }
         size_t bytes() const;
+        bool drop_graphs();  // whether there were any
     };
     std::vector<std::vector<uint32_t>> run(const Batch &src, uint32_t tgt_lang, int max_new, int sync_every,
                                            bool eos_mask, bool use_graph, const Shortlist *sl,
-                                           std::vector<std::vector<float>> *top);
+                                           std::vector<std::vector<float>> *top, bool may_reside = true);
     void evict(const Entry *keep);
     static void trim_graph_memory();
     Model *model_;
@@ -241,11 +244,22 @@ class Model {
     std::unique_ptr<StaticState> new_state(int b, int s, int m, bool logits, bool row_map = false,
                                            const Shortlist *sl = nullptr, bool kv32 = false,
                                            bool resident = false);
-    // Whether a batch-1 greedy state over head `emb` takes the resident launch; its caller
-    // holds the device's one turn for it (GraphCache::run) and decodes again without it when
-    // st.res_flag was raised (drop_resident).
+    // Whether a batch-1 greedy state over head `emb` can take the resident launch; its caller
+    // holds the device's one turn for it (GraphCache::run) and, when st.res_flag was raised,
+    // decodes again without it.
     bool resident_ok(const DevMatrix &emb, int b, int m, int s) const;
-    void drop_resident() { res_layers_ = nullptr; }
+    bool resident_active() const { return res_layers_ && !res_use.pause; }  // for the model's next call
+    // The resident launches of this model's greedy calls: a launch that could not finish its
+    // waits costs a call its polls, so the next calls do without: 16 of them, twice as many
+    // after each further failure, up to 1024, and none again once a call has succeeded.
+    struct ResidentUse {
+        int64_t calls = 0, redone = 0;  // decoded by it; decoded again after a raised flag
+        int pause = 0, next_pause = 16;
+        void succeeded() { ++calls, next_pause = 16; }
+        void failed() { ++redone, pause = next_pause, next_pause = std::min(2 * next_pause, 1024); }
+    } res_use;
+    void set_resident_spins(uint32_t n) { graphs.drop_graphs(), res_spins_ = n; }  // captured launches keep theirs
+    void reset_resident(StaticState &st);  // the launch's words, epoch and flag as at the start
     // src/model.rs:552-612: one decoder step on fixed buffers.  greedy: argmax +
     // bookkeeping, else logits into st.logits and ++step.
     void step(StaticState &st, bool greedy, int mask_id);

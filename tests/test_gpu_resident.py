@@ -39,6 +39,7 @@ def test_resident_step_matches_oracle(model, preset, d, f):
     token is the oracle's argmax after the same prefix, the winning logits within 2e-3."""
     path = model(preset, d, f)
     gpu, orc = M.Translator.load(path), O.Model(path)
+    calls = 0
     try:
         for n, new in ((1, 5), (7, 9), (70, 72)):
             src = [np.random.default_rng(n + d).integers(4, 1200, n).tolist()]
@@ -47,6 +48,8 @@ def test_resident_step_matches_oracle(model, preset, d, f):
             again = gpu.greedy_top(batch, 1100, new, eos_mask=True)  # the captured graph
             eager = gpu.greedy_top(batch, 1100, new, eos_mask=True, graph=False)
             assert again == (toks, top) == eager
+            calls += 3
+            assert gpu.resident_stats() == {"active": True, "calls": calls, "redone": 0}
             tgt = np.array([[2, 1100] + toks[0][:-1]], np.uint32)
             ref = orc.teacher_forced_logits(src, tgt, kv_f16=True)
             argmax_chain_check(toks, top, ref, tie=4e-3)
@@ -76,6 +79,8 @@ def test_resident_step_equals_per_layer_launches(model, monkeypatch, preset, d, 
             a = on.greedy_top(on.encode_cross(src), 1100, new, eos_mask=True)
             b = off.greedy_top(off.encode_cross(src), 1100, new, eos_mask=True)
             assert a == b, (n, new)
+        assert on.resident_stats() == {"active": True, "calls": 8, "redone": 0}
+        assert off.resident_stats() == {"active": False, "calls": 0, "redone": 0}
     finally:
         on.close()
         off.close()
@@ -83,16 +88,63 @@ def test_resident_step_equals_per_layer_launches(model, monkeypatch, preset, d, 
 
 def test_resident_step_off_and_out_of_polls(model, monkeypatch):
     """MALAGA_RESIDENT_STEP=0 and a launch whose waits run out at once (the flag is raised and
-    the call decodes again per layer) give the same bits."""
+    the call decodes again per layer) give the same bits; the next 16 calls do without the
+    launch, 32 after the second failure, and once it gets its polls again it decodes again."""
     path = model("q4_k_m", 512, 1536)
     src = [np.random.default_rng(3).integers(4, 1200, 11).tolist()]
-    out = {}
-    for name, env in (("on", {}), ("off", {"MALAGA_RESIDENT_STEP": "0"}), ("stuck", {"MALAGA_RESIDENT_SPINS": "0"})):
-        gpu = load(path, monkeypatch, **env)
+    off = load(path, monkeypatch, MALAGA_RESIDENT_STEP="0")
+    want = off.greedy_top(off.encode_cross(src), 1100, 20, eos_mask=True)
+    off.close()
+    gpu = load(path, monkeypatch, MALAGA_RESIDENT_SPINS="0")
+    try:
         batch = gpu.encode_cross(src)
-        out[name] = [gpu.greedy_top(batch, 1100, 20, eos_mask=True) for _ in range(3)]
+
+        def decode(n=1, graph=True):
+            for _ in range(n):
+                assert gpu.greedy_top(batch, 1100, 20, eos_mask=True, graph=graph) == want
+
+        def stats(active, calls, redone):
+            assert gpu.resident_stats() == {"active": active, "calls": calls, "redone": redone}
+
+        decode()
+        stats(False, 0, 1)
+        decode(15)
+        stats(False, 0, 1)
+        decode()
+        stats(True, 0, 1)
+        decode(graph=False)  # out of polls again, the same state and its words used again
+        stats(False, 0, 2)
+        decode(32)
+        stats(True, 0, 2)
+        gpu.lib.mlg_debug_resident_spins(gpu.h, 1 << 16)
+        decode(2)
+        decode(graph=False)
+        stats(True, 3, 2)
+    finally:
         gpu.close()
-    assert out["stuck"] == out["off"] == out["on"]
+
+
+def test_resident_step_after_a_failed_launch(model):
+    """The state of a launch that gave up is used again, with words of that launch's tag in it: a
+    later launch takes none of them for its own."""
+    path = model("q4_k_m", 1024, 2560)
+    src = [np.random.default_rng(5).integers(4, 1200, 30).tolist()]
+    gpu = M.Translator.load(path)
+    try:
+        batch = gpu.encode_cross(src)
+        want = gpu.greedy_top(batch, 1100, 40, eos_mask=True)
+        for failed in range(1, 4):
+            gpu.lib.mlg_debug_resident_spins(gpu.h, 0)
+            assert gpu.greedy_top(batch, 1100, 40, eos_mask=True) == want
+            assert gpu.resident_stats()["redone"] == failed
+            gpu.lib.mlg_debug_resident_spins(gpu.h, 1 << 16)
+            for _ in range(16):
+                assert gpu.greedy_top(batch, 1100, 40, eos_mask=True) == want
+            before = gpu.resident_stats()["calls"]
+            assert gpu.greedy_top(batch, 1100, 40, eos_mask=True) == want
+            assert gpu.resident_stats() == {"active": True, "calls": before + 1, "redone": failed}
+    finally:
+        gpu.close()
 
 
 def test_resident_step_from_several_threads(model):
@@ -120,5 +172,6 @@ def test_resident_step_from_several_threads(model):
     for t in threads:
         t.join(100)
     assert sorted(done) == [(i, True) for i in range(len(ts))]
+    assert sum(t.resident_stats()["calls"] for t in ts) > 0
     for t in ts:
         t.close()
