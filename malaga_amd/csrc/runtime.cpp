@@ -11,6 +11,7 @@
 #include "beam.hpp"
 #include "gguf.hpp"
 #include "quant.hpp"
+#include "resident_turn.hpp"
 
 namespace mlg {
 
@@ -1298,26 +1299,6 @@ std::vector<std::vector<uint32_t>> GraphCache::greedy(const Batch &src, uint32_t
     }
 }
 
-namespace {
-// One resident launch at a time on a device: two that each held part of the CUs would wait
-// for CUs the other holds until their polls run out.  A call that finds the turn taken (a
-// thread with another context) decodes with the per-layer launches.
-struct ResidentTurn {
-    static std::atomic<bool> &taken(int device) {
-        static std::atomic<bool> t[64];
-        return t[device & 63];
-    }
-    int device = -1;
-    bool take(int dev) {
-        if (!taken(dev).exchange(true, std::memory_order_acquire)) device = dev;
-        return device >= 0;
-    }
-    ~ResidentTurn() {
-        if (device >= 0) taken(device).store(false, std::memory_order_release);
-    }
-};
-}  // namespace
-
 std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tgt_lang, int max_new, int sync_every,
                                                    bool eos_mask, bool use_graph, const Shortlist *sl,
                                                    std::vector<std::vector<float>> *top, bool may_reside) {
@@ -1330,12 +1311,12 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     const int b = capture ? int(next_pow2(uint32_t(n))) : n;
     const int kb = b, ks = bucket(src.s, 16, max_m), km = bucket(max_new + 2, 32, max_m);
     ++clock_;
-    ResidentTurn turn;  // until the stream is drained below
+    ResidentTurn turn(m.ctx->device, [s] { (void)hipStreamSynchronize(s); });
     const bool can = m.resident_ok(sl ? sl->head : m.embed, kb, km, ks);
     bool resident = false;
     if (can && may_reside) {
         if (m.res_use.pause > 0) --m.res_use.pause;
-        else resident = turn.take(m.ctx->device);
+        else resident = turn.take();
     }
     Entry *e = nullptr;
     for (auto &it : entries_)
@@ -1434,6 +1415,7 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     uint32_t stuck = 0;
     if (st.resident) check_hip(hipMemcpyAsync(&stuck, st.res_flag, 4, hipMemcpyDeviceToHost, s), "D2H");
     check_hip(hipStreamSynchronize(s), "sync");
+    turn.done();
     if (stuck) {  // the results are void
         m.reset_resident(st);
         m.res_use.failed();
