@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <numeric>
+#include <optional>
 #include <type_traits>
 
 #include "beam.hpp"
@@ -1314,6 +1315,8 @@ std::vector<std::vector<uint32_t>> GraphCache::run(const Batch &src, uint32_t tg
     ResidentTurn turn(m.ctx->device, [s] { (void)hipStreamSynchronize(s); });
     const bool can = m.resident_ok(sl ? sl->head : m.embed, kb, km, ks);
     bool resident = false;
+    std::optional<OtherDecode> other;
+    if (!can) other.emplace(m.ctx->device);
     if (can && may_reside) {
         if (m.res_use.pause > 0) --m.res_use.pause;
         else resident = turn.take();
@@ -1445,6 +1448,7 @@ std::vector<std::vector<uint32_t>> Model::beam(const Batch &src, uint32_t tgt_la
         fail(ERR_INVALID, "beam: max_new " + std::to_string(max_new) + " outside 0.." +
                               std::to_string(cfg.max_position_embeddings - 2) + " or beam size < 1");
     ensure_embed();
+    const OtherDecode running(ctx->device);
     hipStream_t s = ctx->stream;
     const int b = src.b, bk = b * k, V = cfg.vocab_size;
     const uint32_t eos = uint32_t(cfg.eos_token_id);
@@ -1566,6 +1570,7 @@ std::vector<std::vector<uint32_t>> Model::greedy_generic(const Batch &src, uint3
         fail(ERR_INVALID, "greedy: max_new " + std::to_string(max_new) + " outside 1.." +
                               std::to_string(cfg.max_position_embeddings - 2));
     ensure_embed();
+    const OtherDecode running(ctx->device);
     hipStream_t s = ctx->stream;
     const int b = src.b, mask_id = eos_mask ? cfg.eos_token_id : -1;
     auto st = new_state(b, src.s, max_new + 2, false, false, nullptr, true);

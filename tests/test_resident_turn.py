@@ -1,5 +1,6 @@
 """ResidentTurn (malaga_amd/csrc/resident_turn.hpp): one decode call per device has the resident
-launch, until everything it launched has finished, also where the call fails on the way."""
+launch, until everything it launched has finished, also where the call fails on the way, and
+none while other contexts decode batches there."""
 import subprocess
 from pathlib import Path
 
@@ -11,6 +12,7 @@ PROGRAM = r"""
 #include <thread>
 #include <vector>
 #include "resident_turn.hpp"
+using mlg::OtherDecode;
 using mlg::ResidentTurn;
 
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
@@ -56,6 +58,16 @@ int main() {
     } catch (const std::runtime_error &) {
     }
     CHECK(drains == 1 && held_while_draining && free_for_another(0));
+    // none beside the batches of other contexts on the device
+    {
+        const OtherDecode batch(0);
+        {
+            const OtherDecode beam(0);
+            CHECK(!free_for_another(0) && free_for_another(1));
+        }
+        CHECK(!free_for_another(0));
+    }
+    CHECK(free_for_another(0));
     // several threads: never two at once
     std::atomic<int> in{0}, most{0}, got{0};
     std::vector<std::thread> ts;
