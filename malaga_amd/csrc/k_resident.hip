@@ -422,6 +422,7 @@ struct Gather {
         lds_barrier();
     }
 };
+static_assert(kResMaxF == 16 * kResGather, "plain_gather's largest poll");
 static_assert(kResGatherWaves == 4, "norm adds four waves' sums");
 
 // waves 0..7 of a head's workgroup; six barriers per layer, as head_gather
@@ -591,7 +592,6 @@ __device__ __forceinline__ void plain_dot(const ResArgs &a, ResLds &s) {
 // waves 8..11 of a projection workgroup
 template <int T, int D>
 __device__ __forceinline__ void plain_gather(const ResArgs &a, ResLds &s, Waiter wt) {
-    constexpr int NU = kResMaxF / kResGather;
     const int t = int(threadIdx.x) - 64 * kResWaves, f = a.f, g = blockIdx.x - a.H, ru = f / kResPlain;
     constexpr int rd = D / kResPlain, rq = 3 * rd;
     // A job's results leave in one store of whole 64-byte pieces (at d = 1024): a word stored by
@@ -610,6 +610,15 @@ __device__ __forceinline__ void plain_gather(const ResArgs &a, ResLds &s, Waiter
             for (int k = 1; k < RowsK4<T, 1, D>::kParts; ++k) v += r[k];
             put(p + g * rd + t, v + bias[t], wt.tag);
         }
+    };
+    // words i, i + 256, .. of the FFN's hidden vector, n of them at once
+    auto gather_u = [&](auto nc, const word_t *p, int &i) {
+        constexpr int n = decltype(nc)::value;
+        float u[n];
+        wt.get<n>(p + i, kResGather, u);
+#pragma unroll
+        for (int k = 0; k < n; ++k) s.u[pos_k6(i + k * kResGather, f / 64)] = u[k];
+        i += n * kResGather;
     };
     Gather<D> gt(t, s.u);
     float4 g1 = gt.vec(s.layers[0].attn_norm.g), b1 = gt.vec(s.layers[0].attn_norm.b), g2, b2;
@@ -633,18 +642,13 @@ __device__ __forceinline__ void plain_gather(const ResArgs &a, ResLds &s, Waiter
         gt.add(wt, w.cout);
         gt.norm(g2, b2, a.eps, s.red, s.h);
         publish(w.u, ru);
-        if (f == kResMaxF) {
-            float u[NU];
-            wt.get<NU>(w.u + t, kResGather, u);
-#pragma unroll
-            for (int k = 0; k < NU; ++k) s.u[pos_k6(t + k * kResGather, f / 64)] = u[k];
-        } else {
-            for (int i = t; i < f; i += kResGather) {
-                float u[1];
-                wt.get<1>(w.u + i, 0, u);
-                s.u[pos_k6(i, f / 64)] = u[0];
-            }
-        }
+        // f / 256 words per thread, whole powers of two polled at once (f is a multiple of 512):
+        // one by one, a step of six layers of FFN 2560 took 152 us, now 136 (3584: 161, 139)
+        int i = t;
+        static_for<0, 4>([&](auto jc) {
+            constexpr int n = 16 >> decltype(jc)::value;
+            if (f & (n * kResGather)) gather_u(std::integral_constant<int, n>{}, w.u, i);
+        });
         lds_barrier();
         publish(w.down, rd);
         if (l + 1 == a.L && t < rd) a.y[g * rd + t] = s.res[t];

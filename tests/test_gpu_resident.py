@@ -66,7 +66,7 @@ def load(path, monkeypatch, **env):
 
 
 @pytest.mark.parametrize("preset", ["q4_k_m", "q5_k_m"])
-@pytest.mark.parametrize("d,f", [(256, 512), (512, 1536), (1024, 4096), (1024, 2560)])
+@pytest.mark.parametrize("d,f", [(256, 512), (512, 1536), (1024, 4096), (1024, 2560), (256, 3584)])
 def test_resident_step_equals_per_layer_launches(model, monkeypatch, preset, d, f):
     """Tokens and winning logits bit for bit, with one key, keys on both sides of the attention's
     groups of 8 and rounds of 64 in both attentions, and several rounds: the sums have one
