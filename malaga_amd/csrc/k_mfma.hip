@@ -179,22 +179,29 @@ __device__ __forceinline__ void block_mfma(const typename MW<T>::Regs (&cur)[WT]
                 if constexpr (W::FOLD) bh[j] = W::b_fold_mid(cur[j], fp[j], s);
                 else W::b_split(cur[j], s, bh[j], bl[j]);
             }
+            if constexpr (W::SPLIT) {  // tile by tile: a fragment of A is done with after its three products
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+                for (int mt = 0; mt < MT; ++mt) {
+                    const h8_t ah = ahs[s & 1][mt], al = als[s & 1][mt];
 #pragma unroll
-                for (int j = 0; j < WT; ++j)
-                    cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahs[s & 1][mt], bh[j], s ? cb[j][mt] : zero, 0, 0, 0);
+                    for (int j = 0; j < WT; ++j)
+                        cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[j], s ? cb[j][mt] : zero, 0, 0, 0);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+                    for (int j = 0; j < WT; ++j) cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[j], cb[j][mt], 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < WT; ++j)
-                    cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(als[s & 1][mt], bh[j], cb[j][mt], 0, 0, 0);
-            if constexpr (W::SPLIT) {
+                    for (int j = 0; j < WT; ++j) cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[j], cb[j][mt], 0, 0, 0);
+                }
+            } else {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                     for (int j = 0; j < WT; ++j)
-                        cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahs[s & 1][mt], bl[j], cb[j][mt], 0, 0, 0);
+                        cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahs[s & 1][mt], bh[j], s ? cb[j][mt] : zero, 0, 0, 0);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int j = 0; j < WT; ++j)
+                        cb[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(als[s & 1][mt], bh[j], cb[j][mt], 0, 0, 0);
             }
         } else {
             float sc[WT], mn[WT];
@@ -303,8 +310,14 @@ constexpr size_t mfma_lds() {
 // MODE 0 stores Y (or split-K partials); MODE 1 (the greedy LM head of 33..64 rows) keeps
 // a (value, lowest index) argmax per X row and workgroup instead (gridDim.y = z = 1).
 // TL: W from the tile-major copy a.w.t (q6_K / q4_K).
+// Waves per SIMD that the kernel is scheduled for: what its LDS leaves room for.  It is
+// dynamic, so the compiler cannot see that, and for the 3 or 4 that its registers would
+// allow it kept the reads of A close to their use (q6_K 1024 x 4096 at 2048 rows 65.9 ->
+// 65.2 us, q8_0 2048 x 2048 at 512 rows 29.6 -> 27.1, q4_K 3072 x 1024 at 911 25.5 -> 24.9).
+constexpr int mfma_waves(int bm) { return bm == 64 ? 2 : 4; }
 template <int T, int BM, int NW, int WT, bool TL, int MODE = 0>
-__global__ __launch_bounds__(NW * 64, 2) void k_mfma(MfmaArgs a) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(mfma_waves(BM), mfma_waves(BM)))) void k_mfma(
+    MfmaArgs a) {
     using W = MW<T>;
     constexpr int MT = BM / 16;
     constexpr int NTH = NW * 64;
