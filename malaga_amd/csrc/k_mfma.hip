@@ -449,15 +449,21 @@ struct Tile {
 // where at least 96 such tiles, or those times the K steps that can be split off (split_k),
 // keep the device busy, else 64 columns.  Measured (us, 256 / 64 columns): q4_K 8192 x 2048 at
 // 1651 rows 159 / 192, q6_K 1024 x 4096 at 911 rows 38.8 / 43.6; below the line q4_K 1024 x 1024
-// at 911 rows 17.1 / 15.9.  K is split only where 64-column tiles alone leave CUs idle: the
-// context's workspace is shared by its streams, and products that fill the device without it
-// (q4_K 4096 x 1024 at 203 rows: 13.7 split / 14.2) stay independent of each other.
+// at 911 rows 17.1 / 15.9.  (Just 256 pieces in 16 splits: q6_K 1024 x 4096 at 203 rows 18.2,
+// in 8 of 64 columns 15.9; in 8 or 32 splits the wide tiles are as good or better.)  A product
+// is split only where it has fewer than 256 tiles of 64
+// columns, or 96 to 128 of 256 (two halves then beat both the unsplit wide tiles and, from K =
+// 2048, the narrow ones: q4_K 2048 x 2048 at 832 rows 29.0 / 38.2 / 31.7 us): the context's
+// workspace holds one product's planes at a time, and the others stay independent of it
+// (q4_K 4096 x 1024 at 203 rows: 13.7 split / 14.2).
 Tile tile_of(const DevMatrix &w, int M) {
     if (M <= 16) return {16, 4, 1};
     if (M <= 32) return {32, 4, 1};
     const Tile wide{64, 8, 2}, narrow{64, 4, 1};
     const int nw = wide.blocks(w.N, M);
-    return nw >= 96 || (narrow.blocks(w.N, M) < 256 && int64_t(nw) * (w.K / kStep) >= 256) ? wide : narrow;
+    const int64_t pieces = int64_t(nw) * (w.K / kStep);
+    const bool split = narrow.blocks(w.N, M) < 256 && (pieces > 256 || (pieces == 256 && nw != 16));
+    return nw >= 96 || split ? wide : narrow;
 }
 
 template <int T, int BM, int NW, int WT, bool TL, int MODE = 0>
@@ -554,15 +560,30 @@ __global__ __launch_bounds__(256) void k_splitk_qkv(const float *part, int ks, i
     }
 }
 
-// K splits that fill the device, within the workspace: the 64-row tiles as many as fit in one
-// resident round (one workgroup of 8 waves per CU, two of 4; one split more would start a
-// second round: q6_K 1024 x 4096 at 911 rows 39.6 us with 300 workgroups, 33.4 with 240), the
-// small ones to at least one workgroup per CU
+// K splits that fill the device, within the workspace.  The small tiles: at least one
+// workgroup per CU.  The 64-row tiles: what 256 workgroups allow, but one or two steps of K
+// per workgroup in the fewest splits that have no more: each adds a plane to write and read
+// (q6_K 1024 x 1024 at 300 rows 11.1 us in 2 splits, 11.7 in 3, 11.3 in 4, 14.4 unsplit; 1024
+// x 4096 at 300 rows, wide, 19.6 in 8 splits, 23.4 in 12).  A second workgroup of 4 waves on a
+// CU only where chains of 3 or more steps are left (512 x 2048 at 832 rows: 17.1 us with 416
+// workgroups of 2 steps, 21.3 with 208 of 4; but 1024 x 1024 at 512 rows: 13.4 with 512 of 1
+// step, 12.3 with 256 of 2).
 int split_k(const DevMatrix &w, int M, size_t ws_bytes) {
     const Tile t = tile_of(w, M);
     const int base = t.blocks(w.N, M), nsteps = w.K / kStep;
-    const int fill = t.bm < 64 ? (256 + base - 1) / base : (t.nw == 8 ? 256 : 512) / base;
-    int ks = base >= 256 ? 1 : std::max(1, std::min(nsteps, fill));
+    auto ceil_div = [](int a, int b) { return (a + b - 1) / b; };
+    int ks = 1;
+    if (base < 256 && t.bm < 64) {
+        ks = std::min(nsteps, ceil_div(256, base));
+    } else if (base < 256) {
+        ks = std::min(nsteps, 256 / base);
+        int s = ceil_div(nsteps, ks);
+        if (t.nw == 4 && s >= 3 && ks > 1) {
+            ks = std::min(nsteps, 512 / base);
+            s = std::max(2, ceil_div(nsteps, ks));
+        }
+        if (s <= 2) ks = ceil_div(nsteps, s);
+    }
     while (ks > 1 && size_t(ks) * M * w.N * sizeof(float) > ws_bytes) --ks;
     return ks;
 }

@@ -148,10 +148,12 @@ def test_gemm_wide_tiles(ctx, t, N, K):
 
 
 @pytest.mark.parametrize("t", (Q4_K, Q5_K, Q6_K, Q8_0, F16))
-@pytest.mark.parametrize("M_,N,K", [(33, 16, 256), (65, 255, 512), (129, 257, 1024), (64, 8192, 256), (127, 4100, 512)])
+@pytest.mark.parametrize("M_,N,K", [(33, 16, 256), (65, 255, 512), (129, 257, 1024), (64, 8192, 256), (127, 4100, 512),
+                                    (300, 1000, 1024), (65, 3000, 2048)])
 def test_gemm_tile_edges(ctx, t, M_, N, K):
     """One row or column past and short of the 64-row / 256- and 64-column tiles, on both sides
-    of the tile rule and with K split or not; the k-quant mins and the centred quants (a MFMA
+    of the tile rule and with K split or not (the last two: in 2 of 4 steps for 160 workgroups,
+    in 4 of 8 for 376); the k-quant mins and the centred quants (a MFMA
     over the sub-block averages of x) also with same-sign activations near the top of the f16
     range, whose sums of 32 are beyond it."""
     rng = np.random.default_rng(M_ + N + t)
