@@ -620,6 +620,7 @@ struct RxArgs {
     float *pv;        // MODE 1: partials [M][parts]
     uint32_t *pi;
     int parts;
+    bool nt;          // MODE 1: the weights do not stay in the cache until the next step
 };
 
 // halves per staged X row: 8 mod 64 dwords, where the A reads (16 rows x 4 k-groups of
@@ -932,14 +933,8 @@ hipError_t launch_rx_tl(const RxArgs &a, int M, int grid, hipStream_t st) {
 template <int T, int MODE>
 hipError_t launch_rx(const RxArgs &a, int M, int grid, hipStream_t st) {
     if constexpr (T == GGML_Q6_K || T == GGML_Q4_K) {
-        // The greedy head of the 600M vocabulary (221 MB of tiles) cannot stay in the 256 MB
-        // Infinity Cache beside the layers' 112 MB, and read with ordinary loads it evicts them
-        // once per step: non-temporal, 32 sentences of 32 tokens took 21.66 instead of 22.35
-        // ms.  (Logits are stored by ordinary loads: alone, over and over, they are faster with
-        // what the cache keeps, 67 against 72 us.)
         if constexpr (T == GGML_Q6_K && MODE == 1)
-            if (a.w.t && size_t(a.w.N) * a.w.nb * (kQ6TileBytes / 16) > size_t(32) << 20)
-                return launch_rx_tl<T, MODE, true, true>(a, M, grid, st);
+            if (a.w.t && a.nt) return launch_rx_tl<T, MODE, true, true>(a, M, grid, st);
         if (a.w.t) return launch_rx_tl<T, MODE, true>(a, M, grid, st);
     }
     return launch_rx_tl<T, MODE, false>(a, M, grid, st);
@@ -1051,7 +1046,16 @@ hipError_t gemm_argmax(const DevMatrix &w, const float *X, int ldx, int M, int m
         default: return hipErrorInvalidValue;
         }
     }
+    // A step reads the decoder layers and the head, and what of both exceeds the Infinity Cache
+    // is read from memory again: with ordinary loads the head evicts the layers.  Read
+    // non-temporally it leaves them there, and costs its own share of the cache.  32 sentences,
+    // 32 tokens, ordinary / non-temporal (d = 1024): 12 layers and 221 MB of head (333 MB) 19.05 /
+    // 18.15 ms, 197 MB in all 17.5 / 17.4 (8 sentences 15.3 / 14.8); but 2 layers and 192 MB 5.09 /
+    // 5.42, 151 MB 6.82 / 7.11: so from three quarters of the 256 MB.  (A head by itself, over and
+    // over, is faster with what the cache keeps.)
+    constexpr size_t kCacheKeeps = 192'000'000;
     RxArgs a = rx_args(w, X, ldx, M);
+    a.nt = w.beside > 0 && tile_major_bytes(w.type, w.N, w.K) + w.beside > kCacheKeeps;
     a.mask_id = mask_id;
     a.pv = pv;
     a.pi = pi;

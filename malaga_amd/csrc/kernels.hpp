@@ -23,6 +23,7 @@ struct DevMatrix {
     // q6_K / q4_K matrices: the MFMA GEMMs' copy in tile-major order (layout_tile_major);
     // null elsewhere
     uint8_t *tm = nullptr;
+    size_t beside = 0;  // a model's LM head: bytes of the decoder layers that each step reads too
 };
 
 // Tile-major q6_K / q4_K (the MFMA GEMMs' W operand): per 16-row tile t < ceil(N / 16)

@@ -526,6 +526,11 @@ void Model::load(const std::string &path) {
         check_hip(hipMemcpy(sl->d_ids, sl->ids.data(), size_t(n) * 4, hipMemcpyHostToDevice), "upload");
         shortlists.push_back(std::move(sl));
     }
+    size_t layers = 0;
+    for (const DecLayer &l : dec)
+        for (const Linear *p : {&l.qkv, &l.out, &l.cross_q, &l.cross_out, &l.up, &l.down}) layers += p->w.bytes;
+    embed.beside = layers;
+    for (auto &sl : shortlists) sl->head.beside = layers;
     build_resident();
     check_hip(hipDeviceSynchronize(), "model upload");
 }
