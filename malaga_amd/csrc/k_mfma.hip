@@ -568,7 +568,11 @@ __global__ __launch_bounds__(256) void k_splitk_qkv(const float *part, int ks, i
 // CU only where chains of 3 or more steps are left (512 x 2048 at 832 rows: 17.1 us with 416
 // workgroups of 2 steps, 21.3 with 208 of 4; but 1024 x 1024 at 512 rows: 13.4 with 512 of 1
 // step, 12.3 with 256 of 2).
-int split_k(const DevMatrix &w, int M, size_t ws_bytes) {
+//
+// reduced: the planes are added up by a kernel that runs in any case (launch_split).  Two
+// halves then also where 129 to 255 tiles of 64 columns could do without (q4_K 1024 x 1024 at
+// 911 rows with the residual and LayerNorm 18.2 us, 25.1 unsplit).
+int split_k(const DevMatrix &w, int M, size_t ws_bytes, bool reduced = false) {
     const Tile t = tile_of(w, M);
     const int base = t.blocks(w.N, M), nsteps = w.K / kStep;
     auto ceil_div = [](int a, int b) { return (a + b - 1) / b; };
@@ -583,6 +587,7 @@ int split_k(const DevMatrix &w, int M, size_t ws_bytes) {
             s = std::max(2, ceil_div(nsteps, ks));
         }
         if (s <= 2) ks = ceil_div(nsteps, s);
+        if (reduced && ks == 1 && t.nw == 4) ks = std::min(nsteps, 2);
     }
     while (ks > 1 && size_t(ks) * M * w.N * sizeof(float) > ws_bytes) --ks;
     return ks;
@@ -1117,7 +1122,7 @@ int launch_split(const DevMatrix &w, const float *X, int ldx, int M, hipStream_t
     *err = hipSuccess;
     if (!ws || !gemm_mfma_supported(w) || ldx % 4 || reinterpret_cast<uintptr_t>(X) % 16) return 1;
     if (gemm_rx_supported(w, M) && w.N >= kRxMinRows) return 1;
-    const int ks = split_k(w, M, ws_bytes);
+    const int ks = split_k(w, M, ws_bytes, true);
     if (ks <= 1) return 1;
     MfmaArgs a{};
     a.w = wptr_of(w);
