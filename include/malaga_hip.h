@@ -243,6 +243,9 @@ int64_t mlg_matrix_bytes(const mlg_matrix *w);
 /* QMatMul::forward (src/model.rs:571-607): y[b][N] = x[b][K] W^T (+ bias) (relu). */
 int mlg_gemv(const mlg_matrix *w, const float *x, int b, float *y, const float *bias, int relu, void *stream);
 int mlg_gemv_max_batch(const mlg_matrix *w);
+/* The same for any M.  Products too small to fill the GPU keep partial sums in the context's one
+ * workspace: the mlg_gemm / mlg_gemm_resid calls on matrices of one context are ordered on one
+ * stream (or by events), and not run beside its model's calls. */
 int mlg_gemm(const mlg_matrix *w, const float *x, int M, float *y, const float *bias, int relu, void *stream);
 /* As mlg_gemm, plus a residual: y = x W^T + bias + r (r may be y itself), then relu.
  * The residual adds of EncoderLayer::forward (src/model.rs:150-153) folded into the
