@@ -334,6 +334,8 @@ struct ResLds {
     ResLayer layers[kResMaxLayers];
 };
 
+static_assert(sizeof(ResLds) <= 64 * 1024, "more needs the kernel's LDS limit raised");
+
 // the decoder's input row into xs[0, d) (plain order) by threads 0 .. d / 16 - 1
 template <int ET>
 __device__ __forceinline__ void embed_row(const ResArgs &a, float *xs) {
@@ -720,16 +722,12 @@ const void *kernel_of(int d) {
 const void *resident_kernel(uint32_t proj, int d) {
     return proj == GGML_Q4_K ? kernel_of<GGML_Q4_K>(d) : kernel_of<GGML_Q5_K>(d);
 }
-hipError_t raise_lds(const void *k) {
-    return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(sizeof(ResLds)));
-}
 }  // namespace
 
 bool step_resident_fits(int d, int H, uint32_t proj, int device) {
     int cus = 0, per_cu = 0;
     const void *k = resident_kernel(proj, d);
     return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
-           raise_lds(k) == hipSuccess &&
            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, kResThreads, sizeof(ResLds)) == hipSuccess &&
            cus * per_cu >= H + kResPlain;
 }

@@ -230,7 +230,7 @@ struct MW<GGML_Q5_K> {
         const h8_t av = __builtin_shufflevector(a, a, 0, 1, 0, 1, 0, 1, 0, 1);
         return b(r, s) * av;
     }
-    static constexpr int MID = 16, MID_NA = 1024;
+    static constexpr int MID = 16, MID_NA = 0;  // centred before they are scaled: na is not read
     __device__ static h8_t b_fold_mid(const Regs &r, const FoldPrep &p, int s) {
         const h2_t a = splat_half(p.a[s >> 1], s & 1);
         const h8_t av = __builtin_shufflevector(a, a, 0, 1, 0, 1, 0, 1, 0, 1);
